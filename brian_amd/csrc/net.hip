@@ -455,9 +455,10 @@ std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_hea
     for (int j = 0; j < M; ++j) d << "  x[" << j << "] = t" << j << ";\n";
   }
   d << "}\n";
-  d << "__device__ inline bool lean_spike(const lean_t (&x)[LEAN_M]) { return x[" << g.th_var << "] > ";
-  if (g.th_kind == TH_VAR) d << "x[" << g.th_vtvar << "]";
-  else d << lit(g.vt, f32);
+  d << "__device__ inline bool lean_spike(const lean_t (&x)[LEAN_M]) { return ";
+  if (g.th_kind == TH_NONE) d << "false";   // a group without a threshold never spikes
+  else if (g.th_kind == TH_VAR) d << "x[" << g.th_var << "] > x[" << g.th_vtvar << "]";
+  else d << "x[" << g.th_var << "] > " << lit(g.vt, f32);
   d << "; }\n}\n#include \"" << kernel_header << "\"\n";
   return d.str();
 }

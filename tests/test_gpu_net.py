@@ -534,3 +534,24 @@ def test_lean_kernel_fp32_rate():
     s, _ = h.get_spikes(g)
     rs, _ = net.raster(gid)
     assert abs(len(s) - len(rs)) / len(rs) < 0.05, (len(s), len(rs))
+
+
+@pytest.mark.parametrize("lean", [0, 1])
+def test_group_without_threshold_never_spikes(lean):
+    """A linear group with reset ops and no threshold (NoThreshold,
+    brian/threshold.py:65-75): no spikes recorded, no reset applied, whatever
+    the sign of its variables, on the model-compiled and the table-driven
+    kernels."""
+    from brian_amd._lib import NetHandle
+    h = NetHandle(1e-4, 64)
+    x0 = np.linspace(-1.0, 1.0, 300)
+    g = h.add_group(np.array([x0]))
+    h.set_linear(g, np.array([[0.5]]), np.array([0.0]))
+    h.add_reset_op(g, 0, 0, 7.0)
+    h.record(g, 1 << 12)
+    h.prepare()
+    h.set_tuning("lean", lean)
+    h.run(20)
+    assert h.spike_count(g) == 0
+    np.testing.assert_array_equal(h.get_state(g, 0, 300), x0 * 0.5 ** 20)
+    h.close()
