@@ -93,7 +93,7 @@ struct HostGroup {
   GroupDev dev{};
   JitKernel jit;          // specialised lean sweep for jit_K neurons per thread
   int jit_K = 0;
-  bool jit_lean = false;  // jit holds k_lean (else the table-driven k_sweep)
+  int jit_is = 0;         // which kernel jit holds (JitKind)
   // independent networks laid back to back (bm_net_set_partition): network
   // p holds neurons [part_off[p], part_off[p+1]); the persistent kernel
   // gives each network one workgroup, largest first (part_order)
@@ -315,39 +315,76 @@ bool one_step(const bm_net *net) {
   return false;
 }
 
-// the common shape every specialised kernel handles, refractoriness aside
-bool lean_shape(const HostGroup &g) {
-  if (g.kind != GK_NEURON || g.upd != UPD_LINEAR || g.M < 1 || g.M > 4) return false;
+// what every model-compiled kernel asks of a group besides its update,
+// threshold and refractoriness
+bool lean_base(const HostGroup &g) {
+  if (g.kind != GK_NEURON || g.M < 1) return false;
   if (!g.mons.empty() || g.mod_var >= 0 || g.stp_conn >= 0 || !g.pins.empty() || g.coin) return false;
   if (!g.ssm_vars.empty()) return false;
-  if (g.th_kind == TH_EMPIRICAL || g.th_kind == TH_POISSON || g.ti_nt > 0) return false;
+  if (g.th_kind == TH_POISSON || g.ti_nt > 0) return false;
   if (g.ring_desc.size() > 1) return false;
   if (g.ring_desc.size() == 1 && g.ring_desc[0].kind != RING_COUNT) return false;
   return true;
+}
+
+// the common shape every specialised kernel handles, refractoriness aside
+bool lean_shape(const HostGroup &g) {
+  return lean_base(g) && g.upd == UPD_LINEAR && g.M <= 4 && g.th_kind != TH_EMPIRICAL;
 }
 
 bool fast_eligible(const HostGroup &g) { return lean_shape(g) && g.refr == REFR_NONE; }
 
 // Refractoriness (one period for every neuron, or one per neuron) with at
 // most one reset op, an assignment (Refractoriness clamps that variable:
-// reset.py:311-332), runs on the model-compiled lean kernel only (not on
-// the table-driven, deferred or persistent kernels).
-bool lean_refr_eligible(const bm_net *net, const HostGroup &g) {
-  if (!net->specialize || !net->lean_kernel || !lean_shape(g)) return false;
+// reset.py:311-332).
+bool lean_refr(const HostGroup &g) {
   if (g.refr != REFR_CONST && g.refr != REFR_ARRAY) return false;
   return g.rs_var.empty() || (g.rs_var.size() == 1 && g.rs_op[0] == 0);
 }
 
-// the group runs a kernel compiled at run time (k_lean or the specialised k_sweep)
-bool jit_group(const bm_net *net, const HostGroup &g) {
-  return net->specialize && (fast_eligible(g) || lean_refr_eligible(net, g));
+// A nonlinear model whose bytecode is compiled as C: any program but one so
+// long that compiling it would take longer than interpreting it saves.
+constexpr int PROG_JIT_MAX = 2048;
+bool prog_jit(const bm_net *net, const HostGroup &g) {
+  return net->specialize && g.upd == UPD_PROGRAM && g.M >= 1 && g.prog_ninstr <= PROG_JIT_MAX;
+}
+
+// The widest window a nonlinear model runs on k_lean, whose steps are
+// unrolled: copies of an update of a thousand instructions for each of up to
+// 16 steps do not fit the instruction cache (64 KiB for two compute units),
+// so longer windows run the general kernel with the model compiled in, which
+// loops over its steps.
+constexpr int LEAN_PROG_WMAX = 2;
+
+// Groups that run on the model-compiled lean kernel only (not on the
+// table-driven, deferred or persistent kernels): refractoriness, empirical
+// thresholds, linear models of more than 4 variables and nonlinear models.
+bool lean_only_eligible(const bm_net *net, const HostGroup &g) {
+  if (!net->specialize || !net->lean_kernel || !lean_base(g) || fast_eligible(g)) return false;
+  if (g.refr != REFR_NONE && !lean_refr(g)) return false;
+  if (g.upd == UPD_LINEAR) return g.M <= 8;
+  return prog_jit(net, g) && net->Wcap <= LEAN_PROG_WMAX;
+}
+
+// the kernel compiled at run time a group runs, if any
+enum JitKind {
+  JIT_NONE = 0,
+  JIT_TABLE,    // k_sweep with the group's tables as constants
+  JIT_LEAN,     // k_lean: the model as code
+  JIT_GENERAL   // the general k_sweep with the nonlinear model as code
+};
+JitKind jit_kind(const bm_net *net, const HostGroup &g) {
+  if (!net->specialize) return JIT_NONE;
+  if (fast_eligible(g)) return g.defer || !net->lean_kernel ? JIT_TABLE : JIT_LEAN;
+  if (lean_only_eligible(net, g)) return JIT_LEAN;
+  return prog_jit(net, g) ? JIT_GENERAL : JIT_NONE;
 }
 
 size_t sweep_shmem(bm_net *net, const HostGroup &g, int K, int W);
 
 int group_K(bm_net *net, const HostGroup &g) {
-  if (fast_eligible(g) || lean_refr_eligible(net, g)) return net->K;
   if (g.upd == UPD_PROGRAM) return 1;
+  if (fast_eligible(g) || lean_only_eligible(net, g)) return net->K;
   if (g.upd == UPD_PERNEURON && g.M > 3) return 1;
   // a captured value per listed spike: four neurons per thread only while
   // the largest window's list still fits the LDS
@@ -358,11 +395,17 @@ int group_K(bm_net *net, const HostGroup &g) {
 
 // dynamic LDS of a sweep launch: spike list (u16, padded to 16 bytes), one
 // modulation value per listed spike when the group drives a modulated
-// connection, then the registers of a bytecode program
-size_t sweep_shmem(bm_net *net, const HostGroup &g, int K, int W) {
+// connection
+size_t sweep_list_shmem(bm_net *net, const HostGroup &g, int K, int W) {
   const size_t cap = (size_t)BLOCK * K * std::max(W, 1);
   size_t shmem = (sizeof(uint16_t) * cap + 15) / 16 * 16 + 16;
   if (g.mod_var >= 0 || g.stp_conn >= 0) shmem += cap * net->tsize();
+  return shmem;
+}
+// the same and the registers of an interpreted bytecode program: what a
+// launch shape is admitted by, whether or not the program is compiled
+size_t sweep_shmem(bm_net *net, const HostGroup &g, int K, int W) {
+  size_t shmem = sweep_list_shmem(net, g, K, W);
   if (g.upd == UPD_PROGRAM) shmem += (size_t)g.prog_nregs * BLOCK * net->tsize();
   return shmem;
 }
@@ -397,6 +440,62 @@ std::string lit(double v, bool f32) {
   return f32 ? std::string("(float)(") + buf + ")" : std::string("(") + buf + ")";
 }
 
+// A nonlinear model's bytecode (equations.py) as straight-line C: one local
+// per program register, the instructions in their order with the
+// interpreter's operations (run_program, net_kernels.hpp), no contraction, so
+// the derivatives have the interpreter's bits.  The compiler drops what an
+// output does not need and shares what the scheme's repeated evaluations have
+// in common (an exponential Euler step of 6 variables runs the program 12
+// times); the interpreter evaluates every instruction each time, a switch and
+// three LDS accesses apiece.  4000 Hodgkin-Huxley neurons, FP64, no delays:
+// 506 us a step interpreted, 8.5 compiled.
+std::string prog_prelude(bm_net *net, const HostGroup &g) {
+  const bool f32 = net->precision == 32;
+  std::ostringstream d;
+  const auto r = [](int q) { return "r" + std::to_string(q); };
+  d << "#include \"devcommon.hpp\"\n#define BM_PROG 1\nnamespace bm {\n"
+    << "typedef " << (f32 ? "float" : "double") << " prog_t;\n#define PROG_SCHEME " << g.prog_scheme
+    << "\nconstexpr bool prog_has[" << g.M << "] = {";
+  for (int j = 0; j < g.M; ++j) d << (j ? "," : "") << (g.prog_code[j] >= 0 ? "true" : "false");
+  d << "};\n__device__ __forceinline__ void prog_body(const prog_t (&x)[" << g.M << "], double t, prog_t (&d)["
+    << g.M << "]) {\n#pragma clang fp contract(off)\n";
+  for (int q = 0; q < g.prog_nregs; ++q)
+    d << "  prog_t " << r(q) << " = " << (q < g.M ? "x[" + std::to_string(q) + "]" : std::string("0")) << ";\n";
+  for (int q = 0; q < g.prog_ninstr; ++q) {
+    const int32_t *ins = g.prog_code.data() + g.M + 4 * q;
+    const std::string a = r(ins[2]), b = r(ins[3]);
+    std::string e;
+    switch (ins[0]) {
+      case OP_MOV: e = a; break;
+      case OP_CONST: e = lit(g.prog_consts[ins[2]], f32); break;
+      case OP_ADD: e = a + " + " + b; break;
+      case OP_SUB: e = a + " - " + b; break;
+      case OP_MUL: e = a + " * " + b; break;
+      case OP_DIV: e = a + " / " + b; break;
+      case OP_NEG: e = "-" + a; break;
+      case OP_EXP: e = "exp(" + a + ")"; break;
+      case OP_LOG: e = "log(" + a + ")"; break;
+      case OP_SQRT: e = "sqrt(" + a + ")"; break;
+      case OP_POW: e = "pow(" + a + ", " + b + ")"; break;
+      case OP_ABS: e = "fabs(" + a + ")"; break;
+      case OP_TIME: e = "(prog_t)t"; break;
+      case OP_SIN: e = "sin(" + a + ")"; break;
+      case OP_COS: e = "cos(" + a + ")"; break;
+      case OP_TANH: e = "tanh(" + a + ")"; break;
+      case OP_CLIPLO: e = a + " < " + b + " ? " + b + " : " + a; break;
+      case OP_CLIPHI: e = a + " > " + b + " ? " + b + " : " + a; break;
+      case OP_GT: e = a + " > " + b + " ? (prog_t)1 : (prog_t)0"; break;
+      case OP_LT: e = a + " < " + b + " ? (prog_t)1 : (prog_t)0"; break;
+      default: continue;
+    }
+    d << "  " << r(ins[1]) << " = " << e << ";\n";
+  }
+  for (int j = 0; j < g.M; ++j)
+    d << "  d[" << j << "] = " << (g.prog_code[j] >= 0 ? r(g.prog_code[j]) : std::string("0")) << ";\n";
+  d << "}\n}\n";
+  return d.str();
+}
+
 // The group's model as compile-time code for k_lean (net_lean.hpp): the
 // channel deliveries, reset ops, linear update and threshold of this group
 // with every constant written out.  FP64 keeps the reference's arithmetic
@@ -408,8 +507,10 @@ std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_hea
   const int nring = (int)g.ring_desc.size();
   const int bits = nring ? g.ring_desc[0].bits : 8, sw = nring ? g.ring_desc[0].sw : 0;
   std::ostringstream d;
+  if (g.upd == UPD_PROGRAM) d << prog_prelude(net, g);
   d << "#include \"net_kernels.hpp\"\nnamespace bm {\n"
-    << "typedef " << (f32 ? "float" : "double") << " lean_t;\n#define LEAN_M " << M << "\n#define LEAN_SW " << sw
+    << "typedef " << (f32 ? "float" : "double") << " lean_t;\n#define LEAN_WMAX " << net->Wcap
+    << "\n#define LEAN_EMP " << (g.th_kind == TH_EMPIRICAL ? g.th_period : -1) << "\n#define LEAN_M " << M << "\n#define LEAN_SW " << sw
     << "\n#define LEAN_REFR " << (g.refr == REFR_CONST ? 1 : (g.refr == REFR_ARRAY ? 2 : 0)) << "\n";
   // deliveries in the channel order (Connections, then DelayConnection flushes)
   d << "__device__ inline void lean_deliver(lean_t (&x)[LEAN_M], uint32_t word) {\n";
@@ -428,8 +529,12 @@ std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_hea
     else d << "  x[" << g.rs_var[r] << "] = x[" << g.rs_var[r] << "] + " << v << ";\n";
   }
   d << "}\n";
-  d << "__device__ inline void lean_update(lean_t (&x)[LEAN_M]) {\n";
-  if (!f32) {
+  d << "__device__ inline void lean_update(lean_t (&x)[LEAN_M], int64_t n) {\n";
+  if (g.upd == UPD_PROGRAM) {
+    // t = n dt (Clock._t, brian/clock.py:186)
+    d << "  program_step_code<LEAN_M>(x, (double)n * " << lit(net->dt, false) << " + 0.0, " << lit(net->dt, false)
+      << ");\n";
+  } else if (!f32) {
     // S <- A.S + C as the left fold A[j,0]*S0 + A[j,1]*S1 + ..., then + C[j]
     // (brian/stateupdater.py:413-416 in that order), no contraction
     d << "#pragma clang fp contract(off)\n";
@@ -479,6 +584,12 @@ JitKernel jit_sweep(bm_net *net, const HostGroup &g, int K) {
     ro.push_back(g.rs_op[r]);
     rvv.push_back(g.rs_vvar[r]);
   }
+  const std::string targ = std::string(net->precision == 64 ? "double" : "float") + ", " + std::to_string(g.M) +
+                           ", " + std::to_string(K);
+  if (jit_kind(net, g) == JIT_GENERAL) {
+    const std::string name = "bm::k_sweep<" + targ + ", 1>";
+    return jit_compile(prog_prelude(net, g) + "#include \"net_kernels.hpp\"\n// " + name + "\n", name);
+  }
   BM_REQUIRE(g.chans.size() <= 4 && g.rs_var.size() <= 4, "lean kernel shape out of range");
   std::ostringstream d;
   d << "#define BM_JIT 1\n#define BM_JIT_SW " << sw << "\n#define BM_JIT_BITS " << bits << "\n#define BM_JIT_NCH "
@@ -491,10 +602,8 @@ JitKernel jit_sweep(bm_net *net, const HostGroup &g, int K) {
     << "\n#include \"net_kernels.hpp\"\n";
   // deferred propagation keeps the table-driven specialisation; every other
   // lean group gets its model compiled in (k_lean)
-  const bool lean = !g.defer && net->lean_kernel;
-  const std::string name = lean ? "bm::k_lean<" + std::to_string(K) + ">"
-                                : std::string("bm::k_sweep<") + (net->precision == 64 ? "double" : "float") + ", " +
-                                      std::to_string(g.M) + ", " + std::to_string(K) + ", 0>";
+  const bool lean = jit_kind(net, g) == JIT_LEAN;
+  const std::string name = lean ? "bm::k_lean<" + std::to_string(K) + ">" : "bm::k_sweep<" + targ + ", 0>";
   const std::string src = (lean ? lean_prelude(net, g) : d.str()) + "// " + name + "\n";
   return jit_compile(src, name);
 }
@@ -545,12 +654,13 @@ void ensure_jit(bm_net *net) {
   if (!net->specialize) return;
   for (auto &gp : net->groups) {
     HostGroup &g = *gp;
-    if (g.kind == GK_GENERATOR || !jit_group(net, g)) continue;
+    const JitKind kind = jit_kind(net, g);
+    if (kind == JIT_NONE) continue;
     const int K = group_K(net, g);
-    if (g.jit_K == K && g.jit.fn && g.jit_lean == net->lean_kernel) continue;
+    if (g.jit_K == K && g.jit.fn && g.jit_is == kind) continue;
     g.jit = jit_sweep(net, g, K);
     g.jit_K = K;
-    g.jit_lean = net->lean_kernel;
+    g.jit_is = kind;
   }
 }
 
@@ -776,10 +886,11 @@ void launch_group(bm_net *net, HostGroup &g, int64_t rel0, int W, int skip_first
   const int64_t per_block = (int64_t)BLOCK * K;
   const int64_t blocks = (g.N + per_block - 1) / per_block;
   if (blocks == 0) return;
-  const size_t shmem = sweep_shmem(net, g, K, W);
+  const JitKind kind = jit_kind(net, g);
+  const size_t shmem = kind == JIT_NONE ? sweep_shmem(net, g, K, W) : sweep_list_shmem(net, g, K, W);
   const bool fast = fast_eligible(g);
-  if (jit_group(net, g)) {
-    BM_REQUIRE(g.jit_K == K && g.jit.fn, "specialised sweep kernel not prepared for this shape");
+  if (kind != JIT_NONE) {
+    BM_REQUIRE(g.jit_K == K && g.jit.fn && g.jit_is == kind, "specialised sweep kernel not prepared for this shape");
     void *args[] = {(void *)&g.dev, (void *)&dbase, (void *)&rel0, (void *)&W, (void *)&skip_first_tail,
                     (void *)&tail_only};
     BM_HIP(hipModuleLaunchKernel(g.jit.fn, (unsigned)blocks, 1, 1, BLOCK, 1, 1, (unsigned)shmem, net->stream,

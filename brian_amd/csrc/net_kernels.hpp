@@ -167,6 +167,57 @@ __device__ inline void program_step(const GroupDev &g, T (&s)[M][1], T *reg, int
   }
 }
 
+#ifdef BM_PROG
+// The same step with the program compiled in (prog_body, prog_has and
+// PROG_SCHEME come from the generated source, net.hip:prog_prelude): the
+// operations of program_step in its order.
+template <int M>
+__device__ __forceinline__ void program_step_code(prog_t (&s)[M], double t, double dt64) {
+#pragma clang fp contract(off)
+  const prog_t dt = (prog_t)dt64;
+  if constexpr (PROG_SCHEME == 1 || PROG_SCHEME == 2) {
+    prog_t d1[M];
+    prog_body(s, t, d1);
+    if constexpr (PROG_SCHEME == 1) {
+#pragma unroll
+      for (int j = 0; j < M; ++j)
+        if (prog_has[j]) s[j] = s[j] + dt * d1[j];
+    } else {
+      const prog_t half = (prog_t)0.5 * dt;
+      prog_t mid[M];
+#pragma unroll
+      for (int j = 0; j < M; ++j) mid[j] = prog_has[j] ? s[j] + half * d1[j] : s[j];
+      prog_body(mid, t, d1);
+#pragma unroll
+      for (int j = 0; j < M; ++j)
+        if (prog_has[j]) s[j] = s[j] + dt * d1[j];
+    }
+  } else {
+    prog_t a[M], b[M];
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      if (!prog_has[j]) continue;
+      prog_t x[M], d[M];
+#pragma unroll
+      for (int q = 0; q < M; ++q) x[q] = q == j ? (prog_t)0 : s[q];
+      prog_body(x, t, d);
+      const prog_t b0 = d[j];
+      x[j] = (prog_t)1;
+      prog_body(x, t, d);
+      a[j] = d[j] - b0;
+      b[j] = b0 / a[j];
+    }
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      if (!prog_has[j]) continue;
+      prog_t x = s[j] + b[j];
+      x = x * exp(a[j] * dt);
+      s[j] = x - b[j];
+    }
+  }
+}
+#endif
+
 template <typename T>
 __device__ inline T load_T(const void *p, int64_t i) { return static_cast<const T *>(p)[i]; }
 
@@ -803,7 +854,16 @@ __global__ __launch_bounds__(BLOCK) void k_sweep(const GroupDev g, const int64_t
             T one[MM][1];
 #pragma unroll
             for (int j = 0; j < MM; ++j) one[j][0] = s[j][0];
+#ifdef BM_PROG
+            T x[MM];
+#pragma unroll
+            for (int j = 0; j < MM; ++j) x[j] = one[j][0];
+            program_step_code<MM>(x, t, g.dt);
+#pragma unroll
+            for (int j = 0; j < MM; ++j) one[j][0] = x[j];
+#else
             program_step<T, MM>(g, one, reg, tid, t);
+#endif
 #pragma unroll
             for (int j = 0; j < MM; ++j) s[j][0] = one[j][0];
           }

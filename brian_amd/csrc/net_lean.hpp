@@ -1,7 +1,7 @@
 // Lean sweep kernel compiled at run time (hipRTC) for one group of the
-// common shape: shared linear propagator, at most one packed count ring,
-// reset ops, constant or variable threshold, and optionally
-// Refractoriness with one period for all neurons (LEAN_REFR).
+// common shape: shared linear propagator or a nonlinear model's program, at
+// most one packed count ring, reset ops, constant, variable or empirical
+// threshold, and optionally Refractoriness (LEAN_REFR).
 //
 // The source that includes this header first defines the group's model as
 // compile-time code (generated on the host, net.hip:lean_prelude):
@@ -9,7 +9,14 @@
 //   LEAN_M, LEAN_SW            state variables; ring bytes per neuron (0: none)
 //   lean_deliver(x, word)      applies the channel counts of one ring slice
 //   lean_reset(x)              the reset ops (brian/reset.py:139-147)
-//   lean_update(x)             S <- A.S + C with A and C as literals
+//   lean_update(x, n)          step n: S <- A.S + C with A and C as literals, or
+//                              the integration scheme's step of the program
+//   LEAN_WMAX                  the widest window the network's delays allow: what
+//                              the step loop is unrolled to (a network without
+//                              delays, one step: 7.1 -> 6.4 us a step at 4000
+//                              neurons in FP64 against 16 guarded copies)
+//   LEAN_EMP                   EmpiricalThreshold's period in steps
+//                              (brian/threshold.py:409-457), -1: none
 //   lean_spike(x)              the threshold condition (brian/threshold.py:160-191)
 //   LEAN_REFR                  1: Refractoriness (brian/reset.py:311-332), the
 //                              reset op held while step - last spike < period
@@ -20,7 +27,7 @@
 // so that a step costs only the arithmetic of the model: zero entries of A
 // vanish in FP32, and there are no table lookups.
 //
-// One launch advances W <= WMAX steps (kernel step n runs the tail of step
+// One launch advances W <= LEAN_WMAX steps (kernel step n runs the tail of step
 // n-1 -- deliveries, then the reset of a neuron that spiked at n-1 -- and
 // the head of step n: update and threshold, as k_sweep does).  The ring
 // slices of the whole window are loaded at once and their slots zeroed, the
@@ -33,6 +40,8 @@
 #ifndef LEAN_REFR
 #define LEAN_REFR 0
 #endif
+// the last spike step of each neuron is followed within the window
+#define LEAN_LAST (LEAN_REFR || LEAN_EMP >= 0)
 
 namespace bm {
 
@@ -56,7 +65,7 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
 
   T s[K][M];
   int32_t last[K], last0[K];
-#if LEAN_REFR
+#if LEAN_LAST
   int32_t lastw[K];  // last spike step, advanced step by step within the window
 #endif
 #if LEAN_REFR == 2
@@ -69,7 +78,7 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
     valid[k] = i < N;
     last[k] = valid[k] ? g.last[i] : NEVER;
     last0[k] = last[k];
-#if LEAN_REFR
+#if LEAN_LAST
     lastw[k] = last[k];
 #endif
 #if LEAN_REFR == 2
@@ -80,11 +89,11 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
   }
 
   // ring slices of every step of the window, loaded at once, then zeroed
-  uint32_t cw[WMAX][K];
+  uint32_t cw[LEAN_WMAX][K];
   int slot0 = (int)((n0 - 1) % g.D);
   if (slot0 < 0) slot0 += g.D;
 #pragma unroll
-  for (int u = 0; u < WMAX; ++u) {
+  for (int u = 0; u < LEAN_WMAX; ++u) {
 #pragma unroll
     for (int k = 0; k < K; ++k) cw[u][k] = 0u;
     if constexpr (LEAN_SW > 0) {
@@ -101,7 +110,7 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
   }
   if constexpr (LEAN_SW > 0) {
 #pragma unroll
-    for (int u = 0; u < WMAX; ++u) {
+    for (int u = 0; u < LEAN_WMAX; ++u) {
       if (u < nsteps && !(u == 0 && skip_first_tail)) {
         int sl = slot0 + u;
         if (sl >= g.D) sl -= g.D;
@@ -118,9 +127,9 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
   bool prev[K];                       // spiked at the previous step: reset in this tail
 #pragma unroll
   for (int k = 0; k < K; ++k) prev[k] = valid[k] && last[k] == (int32_t)(n0 - 1);
-  unsigned long long spk[WMAX][K];    // threshold ballot of each step (wavefront-uniform)
+  unsigned long long spk[LEAN_WMAX][K];    // threshold ballot of each step (wavefront-uniform)
 #pragma unroll
-  for (int w = 0; w < WMAX; ++w) {
+  for (int w = 0; w < LEAN_WMAX; ++w) {
 #pragma unroll
     for (int k = 0; k < K; ++k) spk[w][k] = 0ull;
     if (w >= nsteps) continue;
@@ -147,9 +156,12 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
     if (tail_only) continue;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      lean_update(s[k]);
-#if LEAN_REFR
+      lean_update(s[k], n0 + w);
       bool sp = valid[k] && lean_spike(s[k]);
+#if LEAN_EMP >= 0
+      if (lastw[k] != NEVER && (n0 + w) - (int64_t)lastw[k] <= LEAN_EMP) sp = false;
+#endif
+#if LEAN_REFR
       if (sp && lastw[k] != NEVER) {
         // next allowed spike time in seconds, as the generic sweep tests it
         const double t = (double)(n0 + w) * g.dt + 0.0;
@@ -160,9 +172,9 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
         sp = lt + g.refr_time <= t;
 #endif
       }
+#endif
+#if LEAN_LAST
       if (sp) lastw[k] = (int32_t)(n0 + w);
-#else
-      const bool sp = valid[k] && lean_spike(s[k]);
 #endif
       spk[w][k] = __ballot(sp);
       prev[k] = sp;
@@ -172,7 +184,7 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
   // ---------------- spike list of the window (wavefront ballots -> LDS)
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < WMAX; ++w) {
+  for (int w = 0; w < LEAN_WMAX; ++w) {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const unsigned long long mask = spk[w][k];

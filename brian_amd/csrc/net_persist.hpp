@@ -378,7 +378,7 @@ __device__ __attribute__((always_inline)) inline void persist_network(const Grou
     uint32_t nzk = 0u;  // its slots with spikes
 #define PERSIST_HEAD(k, x)                                                                       \
   {                                                                                              \
-    lean_update(x);                                                                              \
+    lean_update(x, n);                                                                           \
     PERSIST_PUT(k, x)                                                                            \
     const bool sp = ((valid >> (k)) & 1u) && lean_spike(x);                                      \
     const unsigned long long mask = __ballot(sp);                                                \

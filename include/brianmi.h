@@ -321,7 +321,9 @@ int bm_net_set_partition(bm_net *net, int gid, int nparts, const int64_t *offset
  *   BM_TUNE_SPECIALIZE         1 (default): the lean sweep kernel of each group
  *                              is compiled at run time (hipRTC) with the group's
  *                              ring layout, channel table, resets and threshold
- *                              as constants; 0: the precompiled generic form
+ *                              as constants, a nonlinear model's program as code;
+ *                              0: the precompiled generic form, programs
+ *                              interpreted
  *   BM_TUNE_DEFER              (before prepare) 1: specialised lean groups
  *                              deliver each window's spikes during the next
  *                              launch, half of the workgroups before and half
