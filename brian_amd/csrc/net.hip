@@ -89,7 +89,7 @@ struct HostGroup {
   std::vector<ChanDev> chans;
   int D = 1;
   int64_t gen_nsteps = 0;
-  int64_t host_raster_read = 0;
+  int64_t raster_first = 0;          // no entry holds an earlier step
   GroupDev dev{};
   JitKernel jit;          // specialised lean sweep for jit_K neurons per thread
   int jit_K = 0;
@@ -191,6 +191,7 @@ struct bm_net {
   int64_t step = 0;       // next step to run
   hipStream_t stream = nullptr;
   DevBuf d_base;          // int64 device step base
+  DevBuf raster_work;     // buffers of the raster sort, as large as the largest raster read so far
   DevBuf hist_ptrs_d, hist_H_d;
   int nhist = 0;
   std::vector<LateModDev> lates;   // modulated Connections with a homogeneous delay
@@ -2659,10 +2660,8 @@ int bm_net_spike_count(bm_net *net, int gid, int64_t *count) {
 }
 
 namespace {
-// The raster's regions gathered on the host (entries step << 32 | index),
-// with the values recorded at spike times when vals is given.
-std::vector<uint64_t> fetch_raster(bm_net *net, HostGroup &g, int64_t cap, std::vector<double> *vals) {
-  const std::vector<unsigned long long> cs = raster_counts(net, g);
+// Total of the regions' counters, none of which may have overflowed.
+int64_t checked_total(HostGroup &g, const std::vector<unsigned long long> &cs) {
   int64_t c = 0;
   for (int r = 0; r < RSHARD; ++r) {
     if ((int64_t)cs[r] > g.raster_region)
@@ -2671,7 +2670,13 @@ std::vector<uint64_t> fetch_raster(bm_net *net, HostGroup &g, int64_t cap, std::
                                     " (record with a larger capacity)");
     c += (int64_t)cs[r];
   }
-  BM_REQUIRE(c <= cap, "output buffer too small");
+  return c;
+}
+
+// The raster's regions gathered on the host (entries step << 32 | index),
+// with the values recorded at spike times when vals is given.
+std::vector<uint64_t> fetch_raster(bm_net *net, HostGroup &g, const std::vector<unsigned long long> &cs, int64_t c,
+                                   std::vector<double> *vals) {
   std::vector<uint64_t> tmp(c);
   const int64_t nv = vals ? (int64_t)g.ssm_vars.size() : 0;
   if (vals) vals->resize((size_t)(c * nv));
@@ -2695,13 +2700,37 @@ int bm_net_get_spikes(bm_net *net, int gid, int32_t *steps, int32_t *idx, int64_
   return guard([&] {
     HostGroup &g = grp(net, gid);
     BM_REQUIRE(g.raster_cap > 0 && net->prepared, "group is not recorded or network not prepared");
-    std::vector<uint64_t> tmp = fetch_raster(net, g, cap, nullptr);
+    const std::vector<unsigned long long> cs = raster_counts(net, g);
+    const int64_t c = checked_total(g, cs);
+    BM_REQUIRE(c <= cap, "output buffer too small");
+    *n_out = c;
+    if (c == 0) return;
+    // sorted on the device, unless its buffers do not fit there
+    const size_t want = raster_sort_bytes(c, g.raster_first, net->step, g.N);
+    bool fits = c < (int64_t(1) << 31);
+    if (fits && net->raster_work.bytes < want) {
+      try {
+        net->raster_work.alloc(want);
+      } catch (const Error &) {
+        (void)hipGetLastError();
+        fits = false;
+      }
+    }
+    if (fits) {
+      launch_raster_sort(g.raster_d.as<unsigned long long>(), g.raster_region, cs.data(), g.raster_first, net->step,
+                         g.N, net->raster_work.p, net->stream);
+      const int32_t *w = net->raster_work.as<int32_t>();
+      BM_HIP(hipMemcpyAsync(steps, w, (size_t)c * 4, hipMemcpyDeviceToHost, net->stream));
+      BM_HIP(hipMemcpyAsync(idx, w + c, (size_t)c * 4, hipMemcpyDeviceToHost, net->stream));
+      BM_HIP(hipStreamSynchronize(net->stream));
+      return;
+    }
+    std::vector<uint64_t> tmp = fetch_raster(net, g, cs, c, nullptr);
     std::sort(tmp.begin(), tmp.end());
     for (size_t q = 0; q < tmp.size(); ++q) {
       steps[q] = (int32_t)(tmp[q] >> 32);
       idx[q] = (int32_t)(tmp[q] & 0xFFFFFFFFu);
     }
-    *n_out = (int64_t)tmp.size();
   });
 }
 
@@ -2727,7 +2756,10 @@ int bm_net_get_spike_states(bm_net *net, int gid, int32_t *steps, int32_t *idx, 
     BM_REQUIRE(g.raster_cap > 0 && net->prepared, "group is not recorded or network not prepared");
     BM_REQUIRE(!g.ssm_vars.empty(), "no variables are recorded at spike times for this group");
     std::vector<double> v;
-    const std::vector<uint64_t> tmp = fetch_raster(net, g, cap, &v);
+    const std::vector<unsigned long long> cs = raster_counts(net, g);
+    const int64_t c = checked_total(g, cs);
+    BM_REQUIRE(c <= cap, "output buffer too small");
+    const std::vector<uint64_t> tmp = fetch_raster(net, g, cs, c, &v);
     const size_t nv = g.ssm_vars.size();
     std::vector<int64_t> order(tmp.size());
     for (size_t q = 0; q < order.size(); ++q) order[q] = (int64_t)q;
@@ -2748,6 +2780,7 @@ int bm_net_clear_spikes(bm_net *net, int gid) {
     BM_REQUIRE(g.raster_cap > 0 && net->prepared, "group is not recorded or network not prepared");
     BM_HIP(hipMemsetAsync(g.raster_count_d.p, 0, (size_t)RSHARD * RSTRIDE * 8, net->stream));
     BM_HIP(hipStreamSynchronize(net->stream));
+    g.raster_first = net->step;
   });
 }
 

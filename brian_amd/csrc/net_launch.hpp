@@ -30,6 +30,14 @@ void launch_advance(int64_t *d_base, int64_t by, hipStream_t st);
 void launch_check_partition(const int64_t *row_ptr, const int32_t *col, int64_t nrows, int64_t src_off,
                             int64_t tgt_off, const int64_t *part_off, int nparts, int *bad, hipStream_t st);
 
+// Sorted raster (raster.hip): `work` (raster_sort_bytes of it) receives n int32
+// steps, then n int32 indices, of the n = sum(counts) entries of the RSHARD
+// regions at base + r * stride, sorted by (step, index).  Steps lie in [first,
+// end), indices in [0, N), and n below 2^31.
+size_t raster_sort_bytes(int64_t n, int64_t first, int64_t end, int64_t N);
+void launch_raster_sort(const unsigned long long *base, int64_t stride, const unsigned long long *counts,
+                        int64_t first, int64_t end, int64_t N, void *work, hipStream_t st);
+
 // block-diagonal random connectivity built on the device (conngen.hip)
 struct GenSpec {
   int kind = 0;                       // 0 block-diagonal Bernoulli, 1 fixed in-degree

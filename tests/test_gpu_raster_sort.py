@@ -1,0 +1,38 @@
+"""Reading a raster sorts it on the device (raster.hip): entries by (step,
+index), repeats kept, at the sizes where the path changes (one workgroup's
+LDS, one tile of the radix sort, several tiles, 64-bit keys), against numpy's
+sort of the generator's table."""
+import numpy as np
+import pytest
+
+from brian_amd._lib import NetHandle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,N,steps", [
+    (0, 10, 50), (1, 1, 1), (2, 1, 3), (3, 300, 4), (63, 20, 40), (1024, 70000, 2), (4095, 1000, 100),
+    (4096, 1000, 100), (4097, 1000, 100), (4097, 40, 4096), (8192, 1 << 20, 700), (50000, 257, 300),
+    (300001, 1 << 20, 2000), (100000, 1 << 20, 5000), (5000, 1 << 22, 40000)])
+def test_raster_is_sorted(n, N, steps):
+    rng = np.random.default_rng(n)
+    s, i = np.sort(rng.integers(0, steps, n)), rng.integers(0, N, n)
+    order = np.lexsort((i, s))
+    s, i = s[order], i[order]
+    h = NetHandle(1e-4, 32)
+    g = h.add_generator(N, s, i)
+    h.record(g, max(n * 64, 1))            # every region may receive all of a window's spikes
+    h.prepare()
+    half = steps // 2
+    h.run(half)
+    a = h.get_spikes(g)
+    np.testing.assert_array_equal(a[0], s[s < half])
+    np.testing.assert_array_equal(a[1], i[s < half])
+    if n % 2:
+        h.clear_spikes(g)                  # later entries only: the keys start at this step
+        s, i = s[s >= half], i[s >= half]
+    h.run(steps - half)
+    b = h.get_spikes(g)
+    np.testing.assert_array_equal(b[0], s)
+    np.testing.assert_array_equal(b[1], i)
+    h.close()
