@@ -496,6 +496,22 @@ def test_pairwise_distance_kernel(n, T):
     np.testing.assert_array_equal(np.diag(D), 0.0)
 
 
+@pytest.mark.parametrize("n,T", [(1, 600), (64, 511), (64, 512), (65, 513), (200, 2049), (513, 300)])
+def test_pairwise_distance_split_samples(n, T):
+    """The samples split over workgroups, at and around the sizes where the
+    number of ranges changes (8 stages of 32 samples) and with a last range
+    that is short: each of the T squares is rounded once per addition, so two
+    orders of summing lie within 2 T eps of each other."""
+    from brian_amd import _lib
+    rng = np.random.default_rng(n + T)
+    X = rng.standard_normal((n, T))
+    D = _lib.pairwise_sq_distance(X, 0.5)
+    ref = 0.5 * ((X[:, None, :] - X[None, :, :]) ** 2).sum(-1) if n < 300 else \
+        0.5 * np.array([((X - x) ** 2).sum(-1) for x in X])
+    np.testing.assert_allclose(D, ref, rtol=2 * T * 2.3e-16)
+    np.testing.assert_array_equal(D, D.T)
+
+
 def test_van_rossum_metric():
     """VanRossumMetric(source, tau) (monitor.py:1378-1486) on three trains
     (one spike at 10 ms, one at 35 ms, none) over 300 ms: the filtered
