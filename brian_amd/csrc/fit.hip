@@ -259,7 +259,7 @@ struct bm_fit {
   bool features = false, record = false;
   DevBuf rec, rec_count;
   int64_t rec_cap = 0;
-  std::vector<double> init_state;     // [nvars][ncand]
+  DevBuf init_state;      // [nvars][ncand], copied to the state when the candidates are set
   std::vector<int32_t> train_start;   // per target: offset of its padded train
   std::vector<int32_t> cand_tgt;
   hipStream_t stream = nullptr;
@@ -341,8 +341,12 @@ __global__ void k_ou_write(T *I, const double *E, const OuArgs o) {
   }
 }
 
+// Buffers keep their memory from one candidate set to the next.
+void size_to(DevBuf &b, size_t bytes) {
+  if (b.bytes != bytes) b.alloc(bytes);
+}
 void upload_scalar(bm_fit *h, DevBuf &b, const double *src, size_t n) {
-  b.alloc(n * h->tsize());
+  size_to(b, n * h->tsize());
   if (!n) return;
   if (h->precision == 64) {
     BM_HIP(hipMemcpyAsync(b.p, src, n * 8, hipMemcpyHostToDevice, h->stream));
@@ -355,7 +359,7 @@ void upload_scalar(bm_fit *h, DevBuf &b, const double *src, size_t n) {
 }
 template <typename R>
 void upload(bm_fit *h, DevBuf &b, const R *src, size_t n) {
-  b.alloc(n * sizeof(R));
+  size_to(b, n * sizeof(R));
   if (!n) return;
   BM_HIP(hipMemcpyAsync(b.p, src, n * sizeof(R), hipMemcpyHostToDevice, h->stream));
   BM_HIP(hipStreamSynchronize(h->stream));
@@ -365,12 +369,14 @@ void upload(bm_fit *h, DevBuf &b, const R *src, size_t n) {
 // coincidence state (next_spike_allowed=1, last_spike_allowed=0 as in
 // gpu_modelfitting.py:364-365), refractoriness.
 void fill_bytes(bm_fit *h, DevBuf &b, size_t n, int byte) {
-  b.alloc(n);
+  size_to(b, n);
   if (n) BM_HIP(hipMemsetAsync(b.p, byte, n, h->stream));
 }
 
 void reset_counters(bm_fit *h) {
-  upload_scalar(h, h->state, h->init_state.data(), h->init_state.size());
+  size_to(h->state, h->init_state.bytes);
+  if (h->state.bytes)
+    BM_HIP(hipMemcpyAsync(h->state.p, h->init_state.p, h->state.bytes, hipMemcpyDeviceToDevice, h->stream));
   const size_t n = (size_t)h->ncand;
   fill_bytes(h, h->spikecount, n * 4, 0);
   fill_bytes(h, h->ncoinc, n * 4, 0);
@@ -451,7 +457,7 @@ int bm_fit_create(int precision, double dt, int ncand, int ntarget, int nvars, i
     }
     upload(h.get(), h->spiketimes, padded.data(), padded.size());
     upload(h.get(), h->train_off, off.data(), off.size());
-    h->init_state.assign((size_t)nvars * ncand, 0.0);
+    fill_bytes(h.get(), h->init_state, (size_t)nvars * ncand * h->tsize(), 0);
     std::vector<int32_t> zeros(ncand, 0);
     upload(h.get(), h->delay, zeros.data(), zeros.size());
     upload(h.get(), h->refr, zeros.data(), zeros.size());
@@ -474,7 +480,7 @@ int bm_fit_set_candidates(bm_fit *h, const double *params, const double *init_st
                           const int32_t *refractory_steps, const int32_t *delay_steps) {
   return guard([&] {
     if (params && h->nparams > 0) upload_scalar(h, h->params, params, (size_t)h->nparams * h->ncand);
-    if (init_state) h->init_state.assign(init_state, init_state + (size_t)h->nvars * h->ncand);
+    if (init_state) upload_scalar(h, h->init_state, init_state, (size_t)h->nvars * h->ncand);
     if (refractory_steps) upload(h, h->refr, refractory_steps, h->ncand);
     if (delay_steps) upload(h, h->delay, delay_steps, h->ncand);
     reset_counters(h);
