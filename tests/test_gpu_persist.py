@@ -68,13 +68,16 @@ def test_persist_queue_overflow_equals_windowed(queue):
         np.testing.assert_array_equal(pst[v], wst[v])
 
 
+@pytest.mark.parametrize("more", [0, 250])
 @pytest.mark.parametrize("prec", [32, 64])
-def test_persist_shape_boundaries(prec):
+def test_persist_shape_boundaries(prec, more):
     """Networks at the edges of the three workgroup shapes (20 neurons per
     thread in FP32, 8 in FP64: 256, 512, 1024 threads), networks smaller
-    than a wavefront, and empty runs between the chunks."""
+    than a wavefront, and empty runs between the chunks; alone (every network
+    on the widest shape) and with more networks than compute units (each on
+    the smallest shape that holds it)."""
     K = 20 if prec == 32 else 8
-    sizes = [1024 * K, 512 * K + 1, 512 * K, 256 * K + 1, 256 * K, 1, 7, 63, 64, 65, 256, 257, 1000]
+    sizes = [1024 * K, 512 * K + 1, 512 * K, 256 * K + 1, 256 * K, 1, 7, 63, 64, 65, 256, 257, 1000] + [30] * more
     d = W.uneven_batch(seed=21, sizes=sizes)
     chunks = (1, 0, 523, 0, 876)
     (ws, wi), wst = _run(d, prec, False, chunks)
