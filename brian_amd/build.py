@@ -34,7 +34,7 @@ def _compile(unit):
     return obj
 
 
-JIT_HEADERS = ["devcommon.hpp", "net_types.hpp", "net_kernels.hpp", "net_lean.hpp", "net_persist.hpp"]
+JIT_HEADERS = ["devcommon.hpp", "net_types.hpp", "net_kernels.hpp", "net_lean.hpp", "net_persist.hpp", "net_small.hpp"]
 JIT_INC = os.path.join(SRC, "jit_src.inc")
 
 

@@ -191,6 +191,9 @@ struct bm_net {
   int64_t step = 0;       // next step to run
   hipStream_t stream = nullptr;
   DevBuf d_base;          // int64 device step base
+  JitKernel small;        // the whole network in one workgroup (net_small.hpp)
+  DevBuf small_d;         // its descriptors, and what they were last copied from
+  std::vector<unsigned char> small_h;
   DevBuf raster_work;     // buffers of the raster sort, as large as the largest raster read so far
   DevBuf hist_ptrs_d, hist_H_d;
   int nhist = 0;
@@ -498,23 +501,12 @@ std::string prog_prelude(bm_net *net, const HostGroup &g) {
   return d.str();
 }
 
-// The group's model as compile-time code for k_lean (net_lean.hpp): the
-// channel deliveries, reset ops, linear update and threshold of this group
-// with every constant written out.  FP64 keeps the reference's arithmetic
-// (count loops, left-fold rows with no contraction); FP32 uses one fused
-// multiply-add per delivery and per non-zero entry of A.
-std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_header = "net_lean.hpp") {
+// The pieces of a group's model as code.
+// Deliveries in the channel order (Connections, then DelayConnection
+// flushes), from one packed count word.
+void emit_deliver(std::ostringstream &d, bm_net *net, const HostGroup &g) {
   const bool f32 = net->precision == 32;
-  const int M = g.M;
-  const int nring = (int)g.ring_desc.size();
-  const int bits = nring ? g.ring_desc[0].bits : 8, sw = nring ? g.ring_desc[0].sw : 0;
-  std::ostringstream d;
-  if (g.upd == UPD_PROGRAM) d << prog_prelude(net, g);
-  d << "#include \"net_kernels.hpp\"\nnamespace bm {\n"
-    << "typedef " << (f32 ? "float" : "double") << " lean_t;\n#define LEAN_WMAX " << net->Wcap
-    << "\n#define LEAN_EMP " << (g.th_kind == TH_EMPIRICAL ? g.th_period : -1) << "\n#define LEAN_M " << M << "\n#define LEAN_SW " << sw
-    << "\n#define LEAN_REFR " << (g.refr == REFR_CONST ? 1 : (g.refr == REFR_ARRAY ? 2 : 0)) << "\n";
-  // deliveries in the channel order (Connections, then DelayConnection flushes)
+  const int bits = g.ring_desc.empty() ? 8 : g.ring_desc[0].bits;
   d << "__device__ inline void lean_deliver(lean_t (&x)[LEAN_M], uint32_t word) {\n";
   const uint32_t mask = bits >= 32 ? 0xFFFFFFFFu : ((1u << bits) - 1u);
   for (const ChanDev &c : g.chans) {
@@ -524,24 +516,29 @@ std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_hea
            << c.is_delay << "); }\n";
   }
   d << "}\n";
-  d << "__device__ inline void lean_reset(lean_t (&x)[LEAN_M]) {\n";
+}
+
+void emit_reset(std::ostringstream &d, bm_net *net, const HostGroup &g, const std::string &head) {
+  d << head << " {\n";
   for (size_t r = 0; r < g.rs_var.size(); ++r) {
-    const std::string v = g.rs_vvar[r] >= 0 ? "x[" + std::to_string(g.rs_vvar[r]) + "]" : lit(g.rs_val[r], f32);
+    const std::string v =
+        g.rs_vvar[r] >= 0 ? "x[" + std::to_string(g.rs_vvar[r]) + "]" : lit(g.rs_val[r], net->precision == 32);
     if (g.rs_op[r] == 0) d << "  x[" << g.rs_var[r] << "] = " << v << ";\n";
     else d << "  x[" << g.rs_var[r] << "] = x[" << g.rs_var[r] << "] + " << v << ";\n";
   }
   d << "}\n";
-  d << "__device__ inline void lean_update(lean_t (&x)[LEAN_M], int64_t n) {\n";
-  if (g.upd == UPD_PROGRAM) {
-    // t = n dt (Clock._t, brian/clock.py:186)
-    d << "  program_step_code<LEAN_M>(x, (double)n * " << lit(net->dt, false) << " + 0.0, " << lit(net->dt, false)
-      << ");\n";
-  } else if (!f32) {
+}
+
+void emit_linear(std::ostringstream &d, bm_net *net, const HostGroup &g, const std::string &head,
+                 const std::string &type) {
+  const int M = g.M;
+  d << head << " {\n";
+  if (net->precision == 64) {
     // S <- A.S + C as the left fold A[j,0]*S0 + A[j,1]*S1 + ..., then + C[j]
     // (brian/stateupdater.py:413-416 in that order), no contraction
     d << "#pragma clang fp contract(off)\n";
     for (int j = 0; j < M; ++j) {
-      d << "  const lean_t t" << j << " = ";
+      d << "  const " << type << " t" << j << " = ";
       for (int q = 0; q < M; ++q) d << (q ? " + " : "") << lit(g.A[j * M + q], false) << " * x[" << q << "]";
       d << ";\n";
     }
@@ -557,16 +554,49 @@ std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_hea
         if (e.empty()) e = (a == 1.0) ? term : lit(a, true) + " * " + term;
         else e = "__builtin_fmaf(" + lit(a, true) + ", " + term + ", " + e + ")";
       }
-      d << "  const lean_t t" << j << " = " << (e.empty() ? "0.0f" : e) << ";\n";
+      d << "  const " << type << " t" << j << " = " << (e.empty() ? "0.0f" : e) << ";\n";
     }
     for (int j = 0; j < M; ++j) d << "  x[" << j << "] = t" << j << ";\n";
   }
   d << "}\n";
-  d << "__device__ inline bool lean_spike(const lean_t (&x)[LEAN_M]) { return ";
+}
+
+void emit_spike(std::ostringstream &d, bm_net *net, const HostGroup &g, const std::string &head) {
+  d << head << " { return ";
   if (g.th_kind == TH_NONE) d << "false";   // a group without a threshold never spikes
   else if (g.th_kind == TH_VAR) d << "x[" << g.th_var << "] > x[" << g.th_vtvar << "]";
-  else d << "x[" << g.th_var << "] > " << lit(g.vt, f32);
-  d << "; }\n}\n#include \"" << kernel_header << "\"\n";
+  else d << "x[" << g.th_var << "] > " << lit(g.vt, net->precision == 32);
+  d << "; }\n";
+}
+
+// The group's model as compile-time code for k_lean (net_lean.hpp): the
+// channel deliveries, reset ops, linear update and threshold of this group
+// with every constant written out.  FP64 keeps the reference's arithmetic
+// (count loops, left-fold rows with no contraction); FP32 uses one fused
+// multiply-add per delivery and per non-zero entry of A.
+std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_header = "net_lean.hpp") {
+  const bool f32 = net->precision == 32;
+  const int M = g.M;
+  const int nring = (int)g.ring_desc.size();
+  const int sw = nring ? g.ring_desc[0].sw : 0;
+  std::ostringstream d;
+  if (g.upd == UPD_PROGRAM) d << prog_prelude(net, g);
+  d << "#include \"net_kernels.hpp\"\nnamespace bm {\n"
+    << "typedef " << (f32 ? "float" : "double") << " lean_t;\n#define LEAN_WMAX " << net->Wcap
+    << "\n#define LEAN_EMP " << (g.th_kind == TH_EMPIRICAL ? g.th_period : -1) << "\n#define LEAN_M " << M << "\n#define LEAN_SW " << sw
+    << "\n#define LEAN_REFR " << (g.refr == REFR_CONST ? 1 : (g.refr == REFR_ARRAY ? 2 : 0)) << "\n";
+  emit_deliver(d, net, g);
+  emit_reset(d, net, g, "__device__ inline void lean_reset(lean_t (&x)[LEAN_M])");
+  if (g.upd == UPD_PROGRAM) {
+    // t = n dt (Clock._t, brian/clock.py:186)
+    d << "__device__ inline void lean_update(lean_t (&x)[LEAN_M], int64_t n) {\n"
+      << "  program_step_code<LEAN_M>(x, (double)n * " << lit(net->dt, false) << " + 0.0, " << lit(net->dt, false)
+      << ");\n}\n";
+  } else {
+    emit_linear(d, net, g, "__device__ inline void lean_update(lean_t (&x)[LEAN_M], int64_t n)", "lean_t");
+  }
+  emit_spike(d, net, g, "__device__ inline bool lean_spike(const lean_t (&x)[LEAN_M])");
+  d << "}\n#include \"" << kernel_header << "\"\n";
   return d.str();
 }
 
@@ -620,7 +650,7 @@ JitKernel jit_compile(const std::string &src, const std::string &name) {
   if (hiprtcCreateProgram(&prog, src.c_str(), "sweep_jit.hip", kJitNumHeaders, kJitHeaders, kJitHeaderNames) !=
       HIPRTC_SUCCESS)
     throw Error(BM_EHIP, "hiprtcCreateProgram failed for the sweep kernel");
-  hiprtcAddNameExpression(prog, name.c_str());
+  if (!name.empty()) hiprtcAddNameExpression(prog, name.c_str());   // else extern "C" k_small
   // packed FP32 instructions stay disabled, as for the rest of the library
   const char *opts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
                         "-packed-fp32-ops"};
@@ -634,8 +664,8 @@ JitKernel jit_compile(const std::string &src, const std::string &name) {
     throw Error(BM_EHIP, "specialised sweep kernel does not compile:\n" + log.substr(0, 4000));
   }
   const char *lowered = nullptr;
-  hiprtcGetLoweredName(prog, name.c_str(), &lowered);
-  const std::string low = lowered ? lowered : "";
+  if (!name.empty()) hiprtcGetLoweredName(prog, name.c_str(), &lowered);
+  const std::string low = name.empty() ? "k_small" : (lowered ? lowered : "");
   size_t sz = 0;
   hiprtcGetCodeSize(prog, &sz);
   std::vector<char> code(sz);
@@ -879,6 +909,257 @@ void run_persist(bm_net *net, int64_t nsteps) {
       net->ev.push_back(b);
       BM_HIP(hipEventRecord(b, net->stream));
     }
+  }
+  net->step += nsteps;
+}
+
+// ---- small networks in one workgroup (net_small.hpp)
+// The largest networks one workgroup advances: 8 neurons per thread in FP64
+// and 16 in FP32 keep the state of 3 variables within the 128 registers of a
+// 1024-thread workgroup (and the rings must fit its LDS: about 15,000 neurons
+// without delays).  us a step, windowed -> here, CUBA network without delays: 1000
+// neurons FP64 4.6 -> 0.8, 4000 6.3 -> 2.0, 8000 6.9 -> 3.9, 8000 with 2000
+// synapses a neuron 15.6 -> 10.6; FP32 12,000 neurons 6.9 -> 3.0; 1000 Poisson
+// inputs with STDP onto 1 neuron 19.2 -> 1.3, onto 64 23.4 -> 2.0.  Beyond
+// 2^24 synapses one compute unit's reads of the rows would bound the step.
+int64_t small_neurons(const bm_net *net) { return net->precision == 32 ? 16384 : 8192; }
+constexpr int64_t SMALL_SYNAPSES = int64_t(1) << 24;
+// Runs of fewer steps keep the windowed kernels: one step takes 25 us either
+// way (launches there, loading and storing the network's state and rings here);
+// 4 steps of 12,000 neurons 50 us windowed, of 4000 neurons 72.
+constexpr int64_t SMALL_MIN_STEPS = 4;
+
+int small_slots(const HostGroup &g) {      // neurons per thread, a power of two
+  int k = 1;
+  while ((int64_t)k * SMALL_THREADS < g.N) k *= 2;
+  return k;
+}
+
+// LDS arrays of the network; returns the bytes in all.
+size_t small_layout(const bm_net *net, SmallNet &sn) {
+  size_t at = 0;
+  const auto take = [&](size_t bytes) {
+    const size_t o = at;
+    at = (at + bytes + 15) / 16 * 16;
+    return (int)o;
+  };
+  std::memset(&sn, 0, sizeof sn);
+  for (size_t gi = 0; gi < net->groups.size(); ++gi) {
+    const HostGroup &g = *net->groups[gi];
+    for (size_t r = 0; r < g.ring_desc.size(); ++r)
+      sn.ring_off[gi][r] = take((size_t)g.D * g.N * (g.ring_desc[r].kind == RING_COUNT ? 4 : net->tsize()));
+    sn.list_off[gi] = take((size_t)g.N * 2);
+    if (g.raster_cap > 0) sn.raster_off[gi] = take((size_t)SMALL_RASTER * 8);
+  }
+  for (size_t s = 0; s < net->stdps.size(); ++s) {
+    const HostConn &c = *net->conns[net->stdps[s]->conn];
+    sn.pre_off[s] = take((size_t)c.src_n * net->tsize());
+    sn.post_off[s] = take((size_t)c.tgt_n * net->tsize());
+  }
+  return at;
+}
+
+// Whether the network runs in one workgroup: networks that otherwise take a
+// launch per step, of Poisson sources and linear neurons that fit it.
+bool small_eligible(const bm_net *net) {
+  if (!net->specialize || !net->lean_kernel || net->Wcap != 1 || net->defer_W > 0) return false;
+  if (net->groups.empty() || net->groups.size() > (size_t)SMALL_GROUPS || net->stdps.size() > (size_t)SMALL_STDP)
+    return false;
+  int64_t N = 0;
+  for (auto &gp : net->groups) {
+    const HostGroup &g = *gp;
+    N += g.N;
+    if (g.N < 1 || N > small_neurons(net)) return false;
+    if (!g.mons.empty() || g.mod_var >= 0 || g.stp_conn >= 0 || !g.pins.empty() || g.coin || !g.ssm_vars.empty() ||
+        g.ti_nt > 0)
+      return false;
+    if (g.kind == GK_POISSON) continue;
+    if (g.kind != GK_NEURON || g.upd != UPD_LINEAR || g.M < 1 || g.M > 4) return false;
+    if (g.th_kind != TH_NONE && g.th_kind != TH_CONST && g.th_kind != TH_VAR) return false;
+    if (g.refr != REFR_NONE && !lean_refr(g)) return false;
+  }
+  int64_t nnz = 0;
+  for (auto &cp : net->conns) {
+    nnz += cp->nnz;
+    if (cp->mod_var >= 0 || cp->stp || nnz > SMALL_SYNAPSES) return false;
+    if (cp->stdp >= 0 && (cp->delay_kind != 0 || cp->hom_delay != 0)) return false;
+  }
+  SmallNet sn;
+  return small_layout(net, sn) <= (size_t)150 * 1024;
+}
+
+// The kernel of one network: its groups' models, its connections and the
+// order of the phases as code.
+std::string small_source(bm_net *net) {
+  const bool f32 = net->precision == 32;
+  const std::string T = f32 ? "float" : "double";
+  std::ostringstream d, o;
+  d << "#include \"net_small.hpp\"\nnamespace bm {\n";
+  const int ng = (int)net->groups.size();
+  for (int gi = 0; gi < ng; ++gi) {
+    HostGroup &g = *net->groups[gi];
+    const int M = g.kind == GK_NEURON ? g.M : 0;
+    const std::string arr = "(T (&x)[" + std::to_string(std::max(M, 1)) + "]";
+    d << "struct SG" << gi << " {\n  using T = " << T << ";\n  static constexpr int GI = " << gi << ", M = " << M
+      << ", K = " << small_slots(g) << ", NRING = " << g.ring_desc.size()
+      << ", REFR = " << (g.refr == REFR_CONST ? 1 : (g.refr == REFR_ARRAY ? 2 : 0))
+      << ";\n  static constexpr bool POISSON = " << (g.kind == GK_POISSON ? "true" : "false")
+      << ";\n  static constexpr bool RCOUNT[4] = {";
+    for (size_t r = 0; r < 4; ++r)
+      d << (r ? "," : "") << (r < g.ring_desc.size() && g.ring_desc[r].kind == RING_COUNT ? "true" : "false");
+    d << "};\n";
+    // the arithmetic of the kernel the group otherwise runs: k_lean's fused
+    // multiply-adds or, in FP32, the general sweep's
+    const bool lean = g.kind == GK_NEURON && jit_kind(net, g) == JIT_LEAN;
+    d << "  static __device__ inline void deliver" << arr << ", const uint32_t (&w)[MAXRING], const T (&f)[MAXRING]) {\n";
+    if (M > 0)
+      for (const ChanDev &c : g.chans) {
+        const RingDev &rd = g.ring_desc[c.ring];
+        const std::string x = "x[" + std::to_string(c.var) + "]";
+        if (rd.kind != RING_COUNT) {
+          d << "    " << x << " = " << x << " + f[" << c.ring << "];\n";
+          continue;
+        }
+        const uint32_t mask = rd.bits >= 32 ? 0xFFFFFFFFu : ((1u << rd.bits) - 1u);
+        const std::string cnt =
+            "((w[" + std::to_string(c.ring) + "] >> " + std::to_string(c.ch * rd.bits) + ") & " + std::to_string(mask) + "u)";
+        if (f32 && lean) d << "    " << x << " = __builtin_fmaf((float)" << cnt << ", " << lit(c.w, true) << ", " << x << ");\n";
+        else d << "    " << x << " = apply_count<T>(" << x << ", " << cnt << ", " << lit(c.w, f32) << ", " << c.is_delay << ");\n";
+      }
+    d << "  }\n";
+    if (M > 0) {
+      emit_reset(d, net, g, "  static __device__ inline void reset" + arr + ")");
+      const std::string head = "  static __device__ inline void update" + arr + ")";
+      if (f32 && !lean) {
+        d << head << " {\n    const T a[" << M * M << "] = {";
+        for (int q = 0; q < M * M; ++q) d << (q ? "," : "") << lit(g.A[q], true);
+        d << "}, c[" << M << "] = {";
+        for (int q = 0; q < M; ++q) d << (q ? "," : "") << lit(g.C[q], true);
+        d << "};\n    T s[" << M << "][1];\n    for (int j = 0; j < M; ++j) s[j][0] = x[j];\n    linear_exact<" << M
+          << ", 1>(s, a, c);\n    for (int j = 0; j < M; ++j) x[j] = s[j][0];\n  }\n";
+      } else {
+        emit_linear(d, net, g, head, "T");
+      }
+      emit_spike(d, net, g, "  static __device__ inline bool spike(const T (&x)[" + std::to_string(M) + "])");
+    }
+    d << "};\n";
+  }
+  // connections in the order of each group's outs
+  std::ostringstream prop;
+  for (int gi = 0; gi < ng; ++gi) {
+    int k = 0;
+    for (size_t ci = 0; ci < net->conns.size(); ++ci) {
+      const HostConn &c = *net->conns[ci];
+      if (c.src != gi) continue;
+      const RingDev &rd = net->groups[c.tgt]->ring_desc[c.ring];
+      // lanes per row: the mean row in one pass where a wavefront holds it
+      int rs = 1;
+      while (rs < 64 && (double)rs * c.src_n < (double)c.nnz) rs *= 2;
+      d << "struct SC" << ci << " {\n  using T = " << T << ";\n  static constexpr int SRC = " << gi << ", TGT = " << c.tgt
+        << ", RING = " << c.ring << ", SHIFT = " << c.ch * rd.bits << ", DLY = " << (c.delay_kind == 1 ? c.dly_bytes : 0)
+        << ", RS = " << rs << ", STDP = " << c.stdp
+        << ";\n  static constexpr bool COUNT = " << (rd.kind == RING_COUNT ? "true" : "false") << ";\n};\n";
+      prop << "    if (S" << gi << " > 0) small_propagate<SC" << ci << ">(gd[" << gi << "].outs[" << k++ << "], "
+           << (c.stdp >= 0 ? "sd + " + std::to_string(c.stdp) : std::string("nullptr")) << ", sm, sn, S" << gi << ", sl"
+           << c.tgt << ", D" << c.tgt << ", N" << c.tgt << ", turn, tid);\n";
+    }
+  }
+  d << "extern \"C\" __global__ __launch_bounds__(SMT) void k_small(const GroupDev *__restrict__ gd, const StdpDev "
+       "*__restrict__ sd, const SmallNet sn, int64_t n0, int nsteps, int skip_first_tail) {\n"
+    << "  extern __shared__ __align__(16) unsigned char sm[];\n  __shared__ int cnt[2 * SMALL_GROUPS];\n"
+    << "  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;\n"
+    << "  if (tid < 2 * SMALL_GROUPS) cnt[tid] = 0;\n";
+  for (int gi = 0; gi < ng; ++gi)
+    d << "  SmallRegs<SG" << gi << "> r" << gi << ";\n  SmallRaster rr" << gi << " = {0, (int)(n0 & 31)};\n  const int D" << gi
+      << " = gd[" << gi << "].D, N" << gi << " = (int)gd[" << gi << "].N;\n  int sl" << gi << " = (int)(n0 % D" << gi
+      << ");\n  small_load<SG" << gi << ">(gd[" << gi << "], r" << gi << ", sm, sn, tid);\n";
+  for (size_t s = 0; s < net->stdps.size(); ++s)
+    d << "  small_traces<" << T << ">(sd[" << s << "], sm, sn, " << s << ", true, tid);\n";
+  d << "  __syncthreads();\n  for (int st = 0; st < nsteps; ++st) {\n    const int64_t n = n0 + st;\n"
+    << "    int *c = cnt + (st & 1) * SMALL_GROUPS;\n    const bool tail = st > 0 || !skip_first_tail;\n";
+  const auto before = [&](int gi) {       // ring slot of step n - 1
+    const std::string i = std::to_string(gi);
+    return "(sl" + i + " == 0 ? D" + i + " - 1 : sl" + i + " - 1)";
+  };
+  for (int gi = 0; gi < ng; ++gi)
+    d << "    small_sweep<SG" << gi << ">(gd[" << gi << "], r" << gi << ", sm, sn, n, tail, " << before(gi) << ", c + " << gi
+      << ", tid);\n";
+  for (size_t s = 0; s < net->stdps.size(); ++s)
+    d << "    small_decay<" << T << ">(sd[" << s << "], sm, sn, " << s << ", tid);\n";
+  d << "    __syncthreads();\n    int turn = 0;\n";
+  for (int gi = 0; gi < ng; ++gi) d << "    const int S" << gi << " = __builtin_amdgcn_readfirstlane(c[" << gi << "]);\n";
+  d << prop.str() << "    if (wv == SMW - 1) {\n";
+  for (int gi = 0; gi < ng; ++gi)
+    if (net->groups[gi]->raster_cap > 0)
+      d << "      small_raster(gd[" << gi << "], sm, sn, " << gi << ", S" << gi << ", n, rr" << gi << ", lane);\n";
+  // the other parity's counts: read last before the barrier above
+  d << "    }\n    if (tid < SMALL_GROUPS) cnt[((st & 1) ^ 1) * SMALL_GROUPS + tid] = 0;\n    __syncthreads();\n";
+  if (!net->stdps.empty()) {
+    std::string any;
+    for (auto &sp : net->stdps) any += (any.empty() ? "S" : " + S") + std::to_string(net->conns[sp->conn]->tgt);
+    d << "    if (" << any << " > 0) {\n";
+    for (size_t s = 0; s < net->stdps.size(); ++s) {
+      const int t = net->conns[net->stdps[s]->conn]->tgt;
+      d << "      small_post<" << T << ">(sd[" << s << "], sm, sn, " << s << ", " << t << ", S" << t << ", tid);\n";
+    }
+    d << "      __syncthreads();\n    }\n";
+  }
+  for (int gi = 0; gi < ng; ++gi) d << "    if (++sl" << gi << " == D" << gi << ") sl" << gi << " = 0;\n";
+  d << "  }\n";
+  for (int gi = 0; gi < ng; ++gi)
+    d << "  small_finish<SG" << gi << ">(gd[" << gi << "], r" << gi << ", sm, sn, n0 + nsteps, " << before(gi) << ", tid);\n";
+  d << "  __syncthreads();\n";
+  for (int gi = 0; gi < ng; ++gi) {
+    d << "  small_store<SG" << gi << ">(gd[" << gi << "], r" << gi << ", sm, sn, tid);\n";
+    if (net->groups[gi]->raster_cap > 0)
+      d << "  if (wv == SMW - 1) small_raster_flush(gd[" << gi
+        << "], reinterpret_cast<unsigned long long *>(sm + sn.raster_off[" << gi << "]), rr" << gi << ", lane);\n";
+  }
+  for (size_t s = 0; s < net->stdps.size(); ++s)
+    d << "  small_traces<" << T << ">(sd[" << s << "], sm, sn, " << s << ", false, tid);\n";
+  d << "}\n}\n";
+  return d.str();
+}
+
+// Compiles (or takes from the cache) the one-workgroup kernel of an eligible
+// network.
+bool ensure_small(bm_net *net) {
+  if (!small_eligible(net)) return false;
+  if (!net->small.fn) net->small = jit_compile(small_source(net), "");
+  return true;
+}
+
+// One run in launches of at most SMALL_CHUNK steps; each applies the tail of
+// its last step.
+constexpr int64_t SMALL_CHUNK = 20000;
+void run_small(bm_net *net, int64_t nsteps) {
+  std::vector<GroupDev> gd;
+  std::vector<StdpDev> sd;
+  for (auto &gp : net->groups) gd.push_back(gp->dev);
+  for (auto &sp : net->stdps) sd.push_back(sp->dev);
+  const size_t gb = gd.size() * sizeof(GroupDev), sb = sd.size() * sizeof(StdpDev);
+  // the descriptors as they stand (rates, tables and raster buffers may change
+  // between runs), copied where they changed
+  std::vector<unsigned char> h(gb + sb);
+  std::memcpy(h.data(), gd.data(), gb);
+  if (sb) std::memcpy(h.data() + gb, sd.data(), sb);
+  if (h != net->small_h) {
+    if (net->small_d.bytes != h.size()) net->small_d.alloc(h.size());
+    net->small_h.clear();
+    BM_HIP(hipMemcpyAsync(net->small_d.p, h.data(), h.size(), hipMemcpyHostToDevice, net->stream));
+    BM_HIP(hipStreamSynchronize(net->stream));
+    net->small_h = std::move(h);
+  }
+  unsigned char *base = net->small_d.as<unsigned char>();
+  SmallNet sn;
+  const size_t lds = small_layout(net, sn);
+  const void *gp = base, *sp = base + gb;
+  for (int64_t done = 0; done < nsteps; done += SMALL_CHUNK) {
+    int64_t n0 = net->step + done;
+    int ns = (int)std::min<int64_t>(SMALL_CHUNK, nsteps - done), skip = 1;
+    void *args[] = {(void *)&gp, (void *)&sp, (void *)&sn, (void *)&n0, (void *)&ns, (void *)&skip};
+    BM_HIP(hipModuleLaunchKernel(net->small.fn, 1, 1, 1, SMALL_THREADS, 1, 1, (unsigned)lds, net->stream, args, nullptr));
+    BM_HIP(hipGetLastError());
   }
   net->step += nsteps;
 }
@@ -1550,6 +1831,7 @@ void prepare(bm_net *net, int window, int K, int use_graph) {
   }
   check_launch_shapes(net);
   ensure_jit(net);
+  (void)ensure_small(net);
   net->d_base.alloc(8);
   int64_t zero = 0;
   BM_HIP(hipMemcpyAsync(net->d_base.p, &zero, 8, hipMemcpyHostToDevice, net->stream));
@@ -1585,6 +1867,10 @@ void run(bm_net *net, int64_t nsteps) {
   if (nsteps == 0) return;
   if (net->persist) {
     run_persist(net, nsteps);
+    return;
+  }
+  if (nsteps >= SMALL_MIN_STEPS && !net->profiling && ensure_small(net)) {
+    run_small(net, nsteps);
     return;
   }
   ensure_jit(net);

@@ -263,4 +263,15 @@ struct StdpDev {
   int64_t ring_slot_bytes;
 };
 
+// One workgroup for a whole small network (net_small.hpp): byte offsets of its
+// LDS arrays.
+constexpr int SMALL_THREADS = 1024;
+constexpr int SMALL_GROUPS = 4, SMALL_STDP = 4;
+constexpr int SMALL_RASTER = 512;     // staged raster entries per recorded group
+struct SmallNet {
+  int ring_off[SMALL_GROUPS][MAXRING];
+  int list_off[SMALL_GROUPS], raster_off[SMALL_GROUPS];
+  int pre_off[SMALL_STDP], post_off[SMALL_STDP];
+};
+
 }  // namespace bm

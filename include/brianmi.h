@@ -323,7 +323,10 @@ int bm_net_set_partition(bm_net *net, int gid, int nparts, const int64_t *offset
  *                              ring layout, channel table, resets and threshold
  *                              as constants, a nonlinear model's program as code;
  *                              0: the precompiled generic form, programs
- *                              interpreted
+ *                              interpreted.  With it (and BM_TUNE_LEAN) runs of 4
+ *                              steps or more of a small network that takes a
+ *                              launch per step (a connection without delay, or
+ *                              STDP) are one launch of one workgroup
  *   BM_TUNE_DEFER              (before prepare) 1: specialised lean groups
  *                              deliver each window's spikes during the next
  *                              launch, half of the workgroups before and half

@@ -1,0 +1,165 @@
+"""Small networks in one workgroup (net_small.hpp) against the windowed
+kernels, which runs of fewer than 4 steps take: the same network run in long
+stretches, and in stretches of at most 3 steps.  Deliveries that are counts:
+rasters and state equal bit for bit; weights per synapse: equal up to the order
+of the floating additions (a handful of values per target and step, so 1e-12
+relative in FP64)."""
+import numpy as np
+import pytest
+
+from brian_amd import workloads as W
+from brian_amd._lib import NetHandle
+from tests.netbuild import cuba_propagator
+
+pytestmark = pytest.mark.gpu
+DT = 1e-4
+
+
+def _csr(rng, nsrc, ntgt, p):
+    m = rng.random((nsrc, ntgt)) < p
+    ptr = np.concatenate([[0], np.cumsum(m.sum(1))])
+    return ptr, np.nonzero(m)[1]
+
+
+def _advance(h, stretches, small):
+    for s in stretches:
+        if small:
+            h.run(s)
+        else:
+            while s > 0:
+                h.run(min(s, 3))
+                s -= min(s, 3)
+
+
+def _both(build, stretches, exact=True, rtol=1e-12):
+    out = []
+    for small in (True, False):
+        h, read = build()
+        _advance(h, stretches, small)
+        out.append(read(h))
+        h.close()
+    assert len(out[0]) == len(out[1])
+    for a, b in zip(*out):
+        if exact or np.issubdtype(np.asarray(a).dtype, np.integer):
+            np.testing.assert_array_equal(a, b)
+        else:
+            np.testing.assert_allclose(a, b, rtol=rtol, atol=rtol * 1e-2)
+    return out[0]
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("n,kind", [
+    (1, "plain"), (63, "plain"), (1025, "plain"), (4000, "plain"), (8192, "plain"), (8193, "plain"), (14900, "plain"), (1000, "refractory"),
+    (1000, "refractory_array"), (2049, "vt"), (700, "delays"), (300, "dense_raster")])
+def test_count_network(n, kind, precision):
+    A, C = cuba_propagator()
+
+    def build():
+        rng = np.random.default_rng(n)
+        ne = max(1, int(0.8 * n))
+        p = min(1.0, 80 / n)
+        S0 = np.zeros((4, n))
+        S0[0] = W.Vr + rng.random(n) * (W.Vt - W.Vr) * (1.0 if kind != "dense_raster" else 3.0)
+        S0[3] = W.Vt + 1e-3 * rng.random(n)
+        AA, CC = np.eye(4), np.zeros(4)
+        AA[:3, :3], CC[:3] = A, C
+        h = NetHandle(DT, precision)
+        g = h.add_group(S0)
+        h.set_linear(g, AA, CC)
+        if kind == "vt":
+            h.set_threshold(g, 0, 0.0, 3)
+            h.add_reset_op(g, 0, 0, W.Vr)
+            h.add_reset_op(g, 3, 1, 1e-3)
+        else:
+            h.set_threshold(g, 0, -0.058 if kind == "dense_raster" else W.Vt)
+            h.add_reset_op(g, 0, 0, W.Vr if kind != "dense_raster" else -0.0579)
+        if kind == "refractory":
+            h.set_refractory(g, 51, 5e-3 - 0.5 * DT)
+        if kind == "refractory_array":
+            r = (1 + 7 * rng.random(n)) * 1e-3
+            h.set_refractory(g, int(r.max() / DT) + 1, r.max() - 0.5 * DT, per_neuron=r)
+        for lo, m, var, w in ((0, ne, 1, W.we), (ne, n - ne, 2, W.wi)):
+            if m == 0:
+                continue
+            ptr, col = _csr(rng, m, n, p)
+            kw = {}
+            if kind == "delays" and var == 1:
+                kw = {"syn_delay": rng.integers(0, 20, len(col)), "max_delay_steps": 20}
+            h.add_connection(g, lo, m, g, 0, n, var, ptr, col, np.full(len(col), w), **kw)
+        h.record(g, 1 << 17)
+        h.prepare()
+        return h, lambda h: [*h.get_spikes(g), *[h.get_state(g, v, n) for v in range(4)]]
+
+    out = _both(build, (2, 300, 1, 4, 250))
+    if n > 1:
+        assert len(out[0]) > 5
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("nin,nout,inter,update", [
+    (1000, 1, 0, 0), (200, 64, 1, 0), (333, 17, 2, 1), (64, 65, 3, 0), (1, 3, 0, 1)])
+def test_poisson_stdp_network(nin, nout, inter, update, precision):
+    """Poisson inputs through plastic weights onto a group, and back from it
+    through fixed weights of their own onto a second group."""
+    d = W.stdp_batch(1, nin)
+
+    def build():
+        rng = np.random.default_rng(nin + nout)
+        h = NetHandle(DT, precision)
+        p = h.add_poisson(nin, 15.0 * (1 + 3 * rng.random(nin)), 7)
+        g = h.add_group(np.vstack([np.full(nout, -0.055), np.zeros(nout)]))
+        h.set_linear(g, d["A"], d["C"])
+        h.set_threshold(g, 0, d["vt"])
+        h.add_reset_op(g, 0, 0, d["vr"])
+        gmax = 10.0 / nin
+        c = h.add_connection(p, 0, nin, g, 0, nout, 1, np.arange(nin + 1) * nout, np.tile(np.arange(nout), nin),
+                             rng.random(nin * nout) * gmax)
+        sid = h.add_stdp(c, d["decay_pre"], d["decay_post"], 0.01 * (gmax if update == 0 else 1),
+                         -0.0105 * (gmax if update == 0 else 1), 0.0, gmax, update, inter)
+        g2 = h.add_group(np.zeros((1, 5)))
+        h.set_linear(g2, np.array([[0.99]]), np.array([0.0]))
+        ptr, col = _csr(rng, nout, 5, 0.5)
+        h.add_connection(g, 0, nout, g2, 0, 5, 0, ptr, col, rng.random(len(col)), delay_steps=2)
+        h.record(g, 1 << 16)
+        h.record(p, 1 << 17)
+        h.set_poisson_rates(p, 100, 200.0 + 0.0 * np.arange(150), False)
+        h.prepare()
+
+        def read(h):
+            return [*h.get_spikes(p), *h.get_spikes(g), h.get_weights(c, nin * nout),
+                    *h.get_stdp_traces(sid, nin, nout), h.get_state(g, 0, nout), h.get_state(g, 1, nout),
+                    h.get_state(g2, 0, 5)]
+        return h, read
+
+    # FP32: the additions of a step in another order, an ulp of 6e-8 each
+    out = _both(build, (3, 400, 7, 500), exact=False, rtol=1e-11 if precision == 64 else 2e-4)
+    assert len(out[0]) > (5 if nin > 1 else 0)
+    if nin >= 64:
+        assert len(out[2]) > 5
+
+
+def test_long_run_and_rate_changes():
+    """A run of more steps than one launch takes, and new rates between
+    runs."""
+    def build():
+        h = NetHandle(DT, 64)
+        p = h.add_poisson(3, np.array([20.0, 30.0, 5.0]), 1)
+        g = h.add_group(np.zeros((1, 2)))
+        h.set_linear(g, np.array([[0.999]]), np.array([0.0]))
+        h.set_threshold(g, 0, 2.0)
+        h.add_reset_op(g, 0, 0, 0.0)
+        h.add_connection(p, 0, 3, g, 0, 2, 0, [0, 2, 4, 6], [0, 1, 0, 1, 0, 1], np.full(6, 0.75))
+        h.record(g, 1 << 14)
+        h.prepare()
+        return h, lambda h: [*h.get_spikes(g), h.get_state(g, 0, 2)]
+    out = []
+    for small in (True, False):
+        h, read = build()
+        _advance(h, (20011,), small)
+        h.set_poisson_base_rates(0, np.array([100.0, 200.0, 0.0]))
+        _advance(h, (2000,), small)
+        out.append(read(h))
+        h.close()
+    assert len(out[0][0]) > 20
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
