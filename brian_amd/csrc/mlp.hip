@@ -85,6 +85,12 @@ struct MlpDev {
 // operand reads aligned and spread rows over the banks
 __host__ __device__ inline int lds_stride(int n) { return n + 8; }
 
+// LDS elements of the dZ1 buffer, which holds the four partial tiles of the
+// output layer's product first
+__host__ __device__ inline int rows_z1(int nh) {
+  return MR * lds_stride(nh) > 4 * MR * NO * 2 ? MR * lds_stride(nh) : 4 * MR * NO * 2;
+}
+
 // One workgroup: rows [r0, r0 + 32) of the batch.  X rows are gathered
 // through idx (FP32 [n][nin]).  TRAIN: loss per row, and the transposed
 // operands of the weight gradients, feature-major with the batch (ldb
@@ -105,7 +111,7 @@ __global__ __launch_bounds__(RT) void k_mlp_rows(const MlpDev m, const float *__
   uint16_t *sA1 = sX + MR * sx;                                // [32][sh]
   uint16_t *sA2 = sA1 + MR * sh;                               // [32][sh], later dZ2
   uint16_t *sZ1 = sA2 + MR * sh;                               // [32][sh] dZ1 (TRAIN)
-  uint16_t *sdO = sZ1 + MR * sh;                               // [32][so]
+  uint16_t *sdO = sZ1 + rows_z1(nh);                           // [32][so]
   float *sO = reinterpret_cast<float *>(sdO + MR * so);        // [32][NO]
   const int r0 = blockIdx.x * MR;
   const int64_t boff = (TRAIN && d_batch) ? *d_batch * (int64_t)B : 0;
@@ -447,7 +453,8 @@ int64_t nparams(const bm_mlp *h) {
 }
 
 size_t rows_shmem(const bm_mlp *h) {
-  return (size_t)MR * (lds_stride(h->ni) + 3 * lds_stride(h->nh) + lds_stride(NO)) * 2 + (size_t)MR * NO * 4;
+  return (size_t)(MR * (lds_stride(h->ni) + 2 * lds_stride(h->nh) + lds_stride(NO)) + rows_z1(h->nh)) * 2 +
+         (size_t)MR * NO * 4;
 }
 
 void drop_graph(bm_mlp *h) {

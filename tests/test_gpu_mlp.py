@@ -51,6 +51,34 @@ def test_mlp_gradient_matches_oracle():
     m.close()
 
 
+@pytest.mark.parametrize("nin,nh,nu,B", [(17, 64, 2, 256), (64, 128, 4, 512), (90, 192, 8, 256), (256, 64, 16, 256),
+                                         (256, 192, 1, 256), (96, 256, 16, 768)])
+def test_mlp_widths_match_oracle(nin, nh, nu, B):
+    """Forward and gradient at every hidden width, with inputs that are not a
+    multiple of 32 and up to 16 outputs: the output layer's partial tiles have
+    LDS of their own at the narrow widths too.  Same tolerances as at 256."""
+    rng = np.random.default_rng(nin + nh)
+    p = L.init_params(nin, nh, nu, seed=3)
+    p = (p + 0.05 * rng.standard_normal(len(p))).astype(np.float32)
+    m = L.MLP(nin, nh, nu, params=p)
+    X = rng.standard_normal((B, nin)).astype(np.float32)
+    U = rng.random((B, nu)).astype(np.float32)
+    Lr, gr = OM.loss_and_grad(p.astype(np.float64), X.astype(np.float64), U.astype(np.float64), nin, nh, nu)
+    loss, g = m.grad(X, U)
+    assert abs(loss - Lr) <= 1e-4 * (1 + abs(Lr))
+    assert np.linalg.norm(g - gr) / np.linalg.norm(gr) < 2e-3
+    loss2, g2 = m.grad(X, U)
+    assert loss2 == loss
+    np.testing.assert_array_equal(g2, g)
+    W1, b1, W2, b2, W3, b3 = OM.unpack(p.astype(np.float64), nin, nh)
+    A1 = OM.bf16(np.maximum(OM.bf16(X) @ OM.bf16(W1) + b1, 0))
+    A2 = OM.bf16(np.maximum(A1 @ OM.bf16(W2) + b2, 0))
+    ref = (A2 @ OM.bf16(W3) + b3)[:, :2 * nu]
+    out = m.forward(X[:B - 5])
+    assert np.max(np.abs(out - ref[:B - 5])) / (1 + np.max(np.abs(ref))) < 2e-3
+    m.close()
+
+
 def test_mlp_training_reduces_loss():
     rng = np.random.default_rng(4)
     n, nin, nu = 8192, 64, 4
