@@ -516,7 +516,7 @@ int bm_mlp_get_params(bm_mlp *h, float *out);
  * capture, serving loops, harnesses that forbid hipMalloc).  X [B][nin],
  * U [B][nu], loss (one float: the mean loss) and grads (nparams floats) are
  * DEVICE pointers; B a multiple of 256 up to 1024, nin <= 128.  The step's
- * buffers live in a fixed scratch array of about 6 MB per GPU held until
+ * buffers live in a fixed scratch array of about 2.4 MB per GPU held until
  * the process ends; the call returns when the results are written.  Calls
  * that overlap on one GPU race on that scratch. */
 int bm_mlp_grad_noalloc(bm_mlp *h, const float *X, const float *U, int B, float *loss, float *grads);
