@@ -1890,46 +1890,36 @@ void run(bm_net *net, int64_t nsteps) {
     if (!net->profiling) return;
     BM_HIP(hipEventRecord(net->ev.back(), net->stream));
   };
-  // first window: the previous run already applied the tail of its last step
-  {
-    const int w = (int)std::min<int64_t>(W, nsteps);
+  // Windows are launched at their offset from the device's step base, which
+  // moves only where captured windows run: a graph's launches hold offsets from
+  // the base at its start.
+  int64_t rel = 0;
+  const auto window = [&](int w, int skip_first_tail) {
     prof_begin();
-    launch_window(net, 0, w, 1);
+    launch_window(net, rel, w, skip_first_tail);
     prof_end();
     check_launch();
-    launch_advance(net->d_base.as<int64_t>(), (int64_t)w, net->stream);
+    rel += w;
     done += w;
-  }
-  const int64_t remaining_windows = (nsteps - done) / W;
-  int64_t wdone = 0;
-  if (net->use_graph && !net->profiling && remaining_windows >= 8) {
-    const int chunk = (int)std::min<int64_t>(remaining_windows, std::max<int64_t>(1, 512 / W));
+  };
+  // first window: the previous run already applied the tail of its last step
+  window((int)std::min<int64_t>(W, nsteps), 1);
+  int64_t windows = (nsteps - done) / W;
+  if (net->use_graph && !net->profiling && windows >= 8) {
+    const int chunk = (int)std::min<int64_t>(windows, std::max<int64_t>(1, 512 / W));
     build_graph(net, chunk);
-    while (remaining_windows - wdone >= chunk) {
+    launch_advance(net->d_base.as<int64_t>(), rel, net->stream);
+    rel = 0;
+    for (; windows >= chunk; windows -= chunk) {
       BM_HIP(hipGraphLaunch(net->graph_exec, net->stream));
-      wdone += chunk;
+      done += (int64_t)chunk * W;
     }
   }
-  for (; wdone < remaining_windows; ++wdone) {
-    prof_begin();
-    launch_window(net, 0, W, 0);
-    prof_end();
-    check_launch();
-    launch_advance(net->d_base.as<int64_t>(), (int64_t)W, net->stream);
-  }
-  done += remaining_windows * W;
-  if (done < nsteps) {
-    const int w = (int)(nsteps - done);
-    prof_begin();
-    launch_window(net, 0, w, 0);
-    prof_end();
-    check_launch();
-    launch_advance(net->d_base.as<int64_t>(), (int64_t)w, net->stream);
-    done += w;
-  }
+  for (; windows > 0; --windows) window(W, 0);
+  if (done < nsteps) window((int)(nsteps - done), 0);
   // tail of the last step: deliveries and resets so the state matches Brian's
   // state after run()
-  for (auto &gp : net->groups) launch_group(net, *gp, 0, 0, 0, 1);
+  for (auto &gp : net->groups) launch_group(net, *gp, rel, 0, 0, 1);
   check_launch();
   net->step += nsteps;
 }
