@@ -321,20 +321,23 @@ bool one_step(const bm_net *net) {
 }
 
 // what every model-compiled kernel asks of a group besides its update,
-// threshold and refractoriness
+// threshold, refractoriness and rings
 bool lean_base(const HostGroup &g) {
-  if (g.kind != GK_NEURON || g.M < 1) return false;
+  if (g.kind != GK_NEURON && g.kind != GK_POISSON) return false;
   if (!g.mons.empty() || g.mod_var >= 0 || g.stp_conn >= 0 || !g.pins.empty() || g.coin) return false;
   if (!g.ssm_vars.empty()) return false;
-  if (g.th_kind == TH_POISSON || g.ti_nt > 0) return false;
-  if (g.ring_desc.size() > 1) return false;
-  if (g.ring_desc.size() == 1 && g.ring_desc[0].kind != RING_COUNT) return false;
-  return true;
+  return g.th_kind != TH_POISSON && g.ti_nt == 0;
+}
+
+// no deliveries, or all of them counts in one packed ring
+bool one_count_ring(const HostGroup &g) {
+  return g.ring_desc.empty() || (g.ring_desc.size() == 1 && g.ring_desc[0].kind == RING_COUNT);
 }
 
 // the common shape every specialised kernel handles, refractoriness aside
 bool lean_shape(const HostGroup &g) {
-  return lean_base(g) && g.upd == UPD_LINEAR && g.M <= 4 && g.th_kind != TH_EMPIRICAL;
+  return lean_base(g) && g.kind == GK_NEURON && g.upd == UPD_LINEAR && g.M >= 1 && g.M <= 4 &&
+         g.th_kind != TH_EMPIRICAL && one_count_ring(g);
 }
 
 bool fast_eligible(const HostGroup &g) { return lean_shape(g) && g.refr == REFR_NONE; }
@@ -361,12 +364,28 @@ bool prog_jit(const bm_net *net, const HostGroup &g) {
 // loops over its steps.
 constexpr int LEAN_PROG_WMAX = 2;
 
+// k_lean holds a whole window's ring slices in registers: one 32-bit word (two
+// for an FP64 float ring) per ring, step and neuron of the thread.  96 of them
+// leave the rest of the step's registers within the 256 of two wavefronts a
+// SIMD; wider ones run the general kernel.  4000 Poisson sources onto 4000
+// neurons through weights and delays of their own, FP32, windows of 6 steps:
+// 4.3 us a step on the general kernels (which load one step's slice at a time and
+// look their tables up each step), 2.5 on k_lean, run and readback together.
+constexpr size_t LEAN_RING_WORDS = 96;
+bool lean_rings(const bm_net *net, const HostGroup &g) {
+  size_t words = 0;
+  for (const RingDev &rd : g.ring_desc) words += rd.kind == RING_COUNT ? 1 : net->tsize() / 4;
+  return one_count_ring(g) || words * net->Wcap * net->K <= LEAN_RING_WORDS;
+}
+
 // Groups that run on the model-compiled lean kernel only (not on the
-// table-driven, deferred or persistent kernels): refractoriness, empirical
-// thresholds, linear models of more than 4 variables and nonlinear models.
+// table-driven, deferred or persistent kernels): several rings or float rings,
+// refractoriness, empirical thresholds, linear models of more than 4 variables,
+// nonlinear models and Poisson sources.
 bool lean_only_eligible(const bm_net *net, const HostGroup &g) {
-  if (!net->specialize || !net->lean_kernel || !lean_base(g) || fast_eligible(g)) return false;
-  if (g.refr != REFR_NONE && !lean_refr(g)) return false;
+  if (!net->specialize || !net->lean_kernel || !lean_base(g) || fast_eligible(g) || !lean_rings(net, g)) return false;
+  if (g.kind == GK_POISSON) return true;
+  if (g.M < 1 || (g.refr != REFR_NONE && !lean_refr(g))) return false;
   if (g.upd == UPD_LINEAR) return g.M <= 8;
   return prog_jit(net, g) && net->Wcap <= LEAN_PROG_WMAX;
 }
@@ -505,6 +524,7 @@ std::string prog_prelude(bm_net *net, const HostGroup &g) {
 // Deliveries in the channel order (Connections, then DelayConnection
 // flushes), from one packed count word.
 void emit_deliver(std::ostringstream &d, bm_net *net, const HostGroup &g) {
+  if (!one_count_ring(g)) return;
   const bool f32 = net->precision == 32;
   const int bits = g.ring_desc.empty() ? 8 : g.ring_desc[0].bits;
   d << "__device__ inline void lean_deliver(lean_t (&x)[LEAN_M], uint32_t word) {\n";
@@ -516,6 +536,31 @@ void emit_deliver(std::ostringstream &d, bm_net *net, const HostGroup &g) {
            << c.is_delay << "); }\n";
   }
   d << "}\n";
+}
+
+// Deliveries from the slices of any rings: the count words w and the float
+// values f of each, in the channel order.  Groups with one count ring keep
+// k_lean's arithmetic (FP32: one fused multiply-add per channel), the others
+// the general sweep's, which they otherwise run.
+void emit_deliver_rings(std::ostringstream &d, bm_net *net, const HostGroup &g, const std::string &head,
+                        const std::string &type) {
+  const bool f32 = net->precision == 32;
+  d << head << " {\n";
+  if (g.kind == GK_NEURON)
+    for (const ChanDev &c : g.chans) {
+      const RingDev &rd = g.ring_desc[c.ring];
+      const std::string x = "x[" + std::to_string(c.var) + "]";
+      if (rd.kind != RING_COUNT) {
+        d << "    " << x << " = " << x << " + f[" << c.ring << "];\n";
+        continue;
+      }
+      const uint32_t mask = rd.bits >= 32 ? 0xFFFFFFFFu : ((1u << rd.bits) - 1u);
+      const std::string cnt =
+          "((w[" + std::to_string(c.ring) + "] >> " + std::to_string(c.ch * rd.bits) + ") & " + std::to_string(mask) + "u)";
+      if (f32 && one_count_ring(g)) d << "    " << x << " = __builtin_fmaf((float)" << cnt << ", " << lit(c.w, true) << ", " << x << ");\n";
+      else d << "    " << x << " = apply_count<" << type << ">(" << x << ", " << cnt << ", " << lit(c.w, f32) << ", " << c.is_delay << ");\n";
+    }
+  d << "  }\n";
 }
 
 void emit_reset(std::ostringstream &d, bm_net *net, const HostGroup &g, const std::string &head) {
@@ -533,7 +578,15 @@ void emit_linear(std::ostringstream &d, bm_net *net, const HostGroup &g, const s
                  const std::string &type) {
   const int M = g.M;
   d << head << " {\n";
-  if (net->precision == 64) {
+  if (net->precision == 32 && !one_count_ring(g)) {
+    // the general sweep's order, which such groups otherwise run
+    d << "  const " << type << " a[" << M * M << "] = {";
+    for (int q = 0; q < M * M; ++q) d << (q ? "," : "") << lit(g.A[q], true);
+    d << "}, c[" << M << "] = {";
+    for (int q = 0; q < M; ++q) d << (q ? "," : "") << lit(g.C[q], true);
+    d << "};\n  " << type << " s[" << M << "][1];\n  for (int j = 0; j < " << M << "; ++j) s[j][0] = x[j];\n  linear_exact<" << M
+      << ", 1>(s, a, c);\n  for (int j = 0; j < " << M << "; ++j) x[j] = s[j][0];\n";
+  } else if (net->precision == 64) {
     // S <- A.S + C as the left fold A[j,0]*S0 + A[j,1]*S1 + ..., then + C[j]
     // (brian/stateupdater.py:413-416 in that order), no contraction
     d << "#pragma clang fp contract(off)\n";
@@ -577,15 +630,29 @@ void emit_spike(std::ostringstream &d, bm_net *net, const HostGroup &g, const st
 std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_header = "net_lean.hpp") {
   const bool f32 = net->precision == 32;
   const int M = g.M;
-  const int nring = (int)g.ring_desc.size();
+  const int nring = g.kind == GK_NEURON ? (int)g.ring_desc.size() : 0;
   const int sw = nring ? g.ring_desc[0].sw : 0;
+  const auto each = [&](auto f) {      // one value per ring, at least one
+    std::string v;
+    for (int r = 0; r < std::max(nring, 1); ++r) v += (r ? "," : "") + std::to_string(r < nring ? f(g.ring_desc[r]) : 0);
+    return v;
+  };
   std::ostringstream d;
   if (g.upd == UPD_PROGRAM) d << prog_prelude(net, g);
   d << "#include \"net_kernels.hpp\"\nnamespace bm {\n"
     << "typedef " << (f32 ? "float" : "double") << " lean_t;\n#define LEAN_WMAX " << net->Wcap
-    << "\n#define LEAN_EMP " << (g.th_kind == TH_EMPIRICAL ? g.th_period : -1) << "\n#define LEAN_M " << M << "\n#define LEAN_SW " << sw
+    << "\n#define LEAN_NRING " << nring << "\n#define LEAN_POISSON " << (g.kind == GK_POISSON ? 1 : 0)
+    << "\nconstexpr int lean_count[] = {" << each([](const RingDev &r) { return r.kind == RING_COUNT ? 1 : 0; })
+    << "}, lean_sw[] = {" << each([](const RingDev &r) { return r.sw; }) << "};\n#define LEAN_EMP " << (g.th_kind == TH_EMPIRICAL ? g.th_period : -1) << "\n#define LEAN_M " << M << "\n#define LEAN_SW " << sw
     << "\n#define LEAN_REFR " << (g.refr == REFR_CONST ? 1 : (g.refr == REFR_ARRAY ? 2 : 0)) << "\n";
+  if (g.kind == GK_POISSON) {
+    d << "}\n#include \"" << kernel_header << "\"\n";
+    return d.str();
+  }
   emit_deliver(d, net, g);
+  emit_deliver_rings(d, net, g, "__device__ inline void lean_deliver_rings(lean_t (&x)[LEAN_M], const uint32_t (&w)[" +
+                     std::to_string(std::max(nring, 1)) + "], const lean_t (&f)[" + std::to_string(std::max(nring, 1)) + "])",
+                     "lean_t");
   emit_reset(d, net, g, "__device__ inline void lean_reset(lean_t (&x)[LEAN_M])");
   if (g.upd == UPD_PROGRAM) {
     // t = n dt (Clock._t, brian/clock.py:186)
@@ -622,7 +689,7 @@ JitKernel jit_sweep(bm_net *net, const HostGroup &g, int K) {
     const std::string name = "bm::k_sweep<" + targ + ", 1>";
     return jit_compile(prog_prelude(net, g) + "#include \"net_kernels.hpp\"\n// " + name + "\n", name);
   }
-  BM_REQUIRE(g.chans.size() <= 4 && g.rs_var.size() <= 4, "lean kernel shape out of range");
+  BM_REQUIRE(g.rs_var.size() <= 4 && (g.chans.size() <= 4 || !one_count_ring(g)), "lean kernel shape out of range");
   std::ostringstream d;
   d << "#define BM_JIT 1\n#define BM_JIT_SW " << sw << "\n#define BM_JIT_BITS " << bits << "\n#define BM_JIT_NCH "
     << g.chans.size() << "\n#define BM_JIT_NRESET " << g.rs_var.size() << "\n#define BM_JIT_NRING " << nring
@@ -1008,38 +1075,11 @@ std::string small_source(bm_net *net) {
     for (size_t r = 0; r < 4; ++r)
       d << (r ? "," : "") << (r < g.ring_desc.size() && g.ring_desc[r].kind == RING_COUNT ? "true" : "false");
     d << "};\n";
-    // the arithmetic of the kernel the group otherwise runs: k_lean's fused
-    // multiply-adds or, in FP32, the general sweep's
-    const bool lean = g.kind == GK_NEURON && jit_kind(net, g) == JIT_LEAN;
-    d << "  static __device__ inline void deliver" << arr << ", const uint32_t (&w)[MAXRING], const T (&f)[MAXRING]) {\n";
-    if (M > 0)
-      for (const ChanDev &c : g.chans) {
-        const RingDev &rd = g.ring_desc[c.ring];
-        const std::string x = "x[" + std::to_string(c.var) + "]";
-        if (rd.kind != RING_COUNT) {
-          d << "    " << x << " = " << x << " + f[" << c.ring << "];\n";
-          continue;
-        }
-        const uint32_t mask = rd.bits >= 32 ? 0xFFFFFFFFu : ((1u << rd.bits) - 1u);
-        const std::string cnt =
-            "((w[" + std::to_string(c.ring) + "] >> " + std::to_string(c.ch * rd.bits) + ") & " + std::to_string(mask) + "u)";
-        if (f32 && lean) d << "    " << x << " = __builtin_fmaf((float)" << cnt << ", " << lit(c.w, true) << ", " << x << ");\n";
-        else d << "    " << x << " = apply_count<T>(" << x << ", " << cnt << ", " << lit(c.w, f32) << ", " << c.is_delay << ");\n";
-      }
-    d << "  }\n";
+    emit_deliver_rings(d, net, g, "  static __device__ inline void deliver" + arr +
+                       ", const uint32_t (&w)[MAXRING], const T (&f)[MAXRING])", "T");
     if (M > 0) {
       emit_reset(d, net, g, "  static __device__ inline void reset" + arr + ")");
-      const std::string head = "  static __device__ inline void update" + arr + ")";
-      if (f32 && !lean) {
-        d << head << " {\n    const T a[" << M * M << "] = {";
-        for (int q = 0; q < M * M; ++q) d << (q ? "," : "") << lit(g.A[q], true);
-        d << "}, c[" << M << "] = {";
-        for (int q = 0; q < M; ++q) d << (q ? "," : "") << lit(g.C[q], true);
-        d << "};\n    T s[" << M << "][1];\n    for (int j = 0; j < M; ++j) s[j][0] = x[j];\n    linear_exact<" << M
-          << ", 1>(s, a, c);\n    for (int j = 0; j < M; ++j) x[j] = s[j][0];\n  }\n";
-      } else {
-        emit_linear(d, net, g, head, "T");
-      }
+      emit_linear(d, net, g, "  static __device__ inline void update" + arr + ")", "T");
       emit_spike(d, net, g, "  static __device__ inline bool spike(const T (&x)[" + std::to_string(M) + "])");
     }
     d << "};\n";

@@ -6,8 +6,10 @@
 // The source that includes this header first defines the group's model as
 // compile-time code (generated on the host, net.hip:lean_prelude):
 //   lean_t                     the arithmetic type (float or double)
-//   LEAN_M, LEAN_SW            state variables; ring bytes per neuron (0: none)
-//   lean_deliver(x, word)      applies the channel counts of one ring slice
+//   LEAN_M                     state variables
+//   LEAN_NRING, lean_count[], lean_sw[]   the rings: counts (else floats), bytes per neuron
+//   lean_deliver_rings(x, w, f)  applies a step's slices of all rings (w count words, f floats)
+//   LEAN_POISSON               1: Poisson sources instead of neurons (no state, no rings)
 //   lean_reset(x)              the reset ops (brian/reset.py:139-147)
 //   lean_update(x, n)          step n: S <- A.S + C with A and C as literals, or
 //                              the integration scheme's step of the program
@@ -49,7 +51,7 @@ template <int K>
 __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t *d_base, int64_t rel0, int W,
                                                 int skip_first_tail, int tail_only) {
   using T = lean_t;
-  constexpr int M = LEAN_M;
+  constexpr int M = LEAN_M, MM = LEAN_M > 0 ? LEAN_M : 1, NR = LEAN_NRING > 0 ? LEAN_NRING : 1;
   extern __shared__ __align__(16) unsigned char smem[];
   uint16_t *sh_list = reinterpret_cast<uint16_t *>(smem);   // (w << 12) | local index
   __shared__ int sh_n;
@@ -63,8 +65,11 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
   const int blk0 = blockIdx.x * (BLOCK * K);
   const int nsteps = tail_only ? 1 : W;
 
-  T s[K][M];
+  T s[K][MM];
   int32_t last[K], last0[K];
+#if LEAN_POISSON
+  uint64_t key[K], thr[K];   // counter stream and threshold of each source
+#endif
 #if LEAN_LAST
   int32_t lastw[K];  // last spike step, advanced step by step within the window
 #endif
@@ -84,43 +89,66 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
 #if LEAN_REFR == 2
     rtime[k] = valid[k] ? g.refr_arr[i] : 0.0;
 #endif
+#if LEAN_POISSON
+    key[k] = counter_key(g.seed, (uint64_t)i);
+    thr[k] = valid[k] ? g.pthr[i] : 0u;
+#endif
 #pragma unroll
     for (int j = 0; j < M; ++j) s[k][j] = valid[k] ? static_cast<const T *>(g.S)[(int64_t)j * N + i] : (T)0;
   }
 
   // ring slices of every step of the window, loaded at once, then zeroed
-  uint32_t cw[LEAN_WMAX][K];
+  uint32_t cw[LEAN_WMAX][K][NR];
+  T fw[LEAN_WMAX][K][NR];
+#if LEAN_NRING > 0
   int slot0 = (int)((n0 - 1) % g.D);
   if (slot0 < 0) slot0 += g.D;
 #pragma unroll
   for (int u = 0; u < LEAN_WMAX; ++u) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) cw[u][k] = 0u;
-    if constexpr (LEAN_SW > 0) {
-      if (u < nsteps && !(u == 0 && skip_first_tail)) {
-        int sl = slot0 + u;
-        if (sl >= g.D) sl -= g.D;
+    for (int k = 0; k < K; ++k) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        cw[u][k][r] = 0u;
+        fw[u][k][r] = (T)0;
+      }
+    }
+    if (u < nsteps && !(u == 0 && skip_first_tail)) {
+      int sl = slot0 + u;
+      if (sl >= g.D) sl -= g.D;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
         const unsigned char *slot =
-            static_cast<const unsigned char *>(g.rings[0].base) + (int64_t)sl * g.rings[0].slot_bytes;
+            static_cast<const unsigned char *>(g.rings[r].base) + (int64_t)sl * g.rings[r].slot_bytes;
 #pragma unroll
-        for (int k = 0; k < K; ++k)
-          if (valid[k]) cw[u][k] = load_slice(slot, blk0 + k * BLOCK + tid, LEAN_SW);
+        for (int k = 0; k < K; ++k) {
+          if (!valid[k]) continue;
+          const int i = blk0 + k * BLOCK + tid;
+          if (lean_count[r]) cw[u][k][r] = load_slice(slot, i, lean_sw[r]);
+          else fw[u][k][r] = reinterpret_cast<const T *>(slot)[i];
+        }
       }
     }
   }
-  if constexpr (LEAN_SW > 0) {
 #pragma unroll
-    for (int u = 0; u < LEAN_WMAX; ++u) {
-      if (u < nsteps && !(u == 0 && skip_first_tail)) {
-        int sl = slot0 + u;
-        if (sl >= g.D) sl -= g.D;
-        unsigned char *slot = static_cast<unsigned char *>(g.rings[0].base) + (int64_t)sl * g.rings[0].slot_bytes;
+  for (int u = 0; u < LEAN_WMAX; ++u) {
+    if (u < nsteps && !(u == 0 && skip_first_tail)) {
+      int sl = slot0 + u;
+      if (sl >= g.D) sl -= g.D;
 #pragma unroll
-        for (int k = 0; k < K; ++k)
-          if (valid[k]) zero_slice(slot, blk0 + k * BLOCK + tid, LEAN_SW);
+      for (int r = 0; r < NR; ++r) {
+        unsigned char *slot = static_cast<unsigned char *>(g.rings[r].base) + (int64_t)sl * g.rings[r].slot_bytes;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          if (!valid[k]) continue;
+          const int i = blk0 + k * BLOCK + tid;
+          if (lean_count[r]) zero_slice(slot, i, lean_sw[r]);
+          else reinterpret_cast<T *>(slot)[i] = (T)0;
+        }
       }
     }
   }
+#endif
   if (tid == 0) sh_n = 0;
 
   // ---------------- the window's steps
@@ -133,10 +161,13 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
 #pragma unroll
     for (int k = 0; k < K; ++k) spk[w][k] = 0ull;
     if (w >= nsteps) continue;
+#if !LEAN_POISSON
     if (!(w == 0 && skip_first_tail)) {
 #pragma unroll
       for (int k = 0; k < K; ++k) {
-        lean_deliver(s[k], cw[w][k]);
+#if LEAN_NRING > 0
+        lean_deliver_rings(s[k], cw[w][k], fw[w][k]);
+#endif
 #if LEAN_REFR
         // the tail of step n0 + w - 1: the reset holds for `period` steps
         // from the spike's own step on
@@ -153,11 +184,21 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
 #endif
       }
     }
+#endif
     if (tail_only) continue;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
+#if LEAN_POISSON
+      // constant rates, or the step's row of a rate table
+      uint64_t t = thr[k];
+      const int64_t row = n0 + w - g.ptab_n0;
+      if (g.ptab && row >= 0 && row < g.ptab_len && valid[k])
+        t = g.ptab[g.ptab_per_neuron ? row * N + (blk0 + k * BLOCK + tid) : row];
+      bool sp = valid[k] && (uint64_t)(uint32_t)(counter_u64(key[k], (uint64_t)(n0 + w)) >> 32) < t;
+#else
       lean_update(s[k], n0 + w);
       bool sp = valid[k] && lean_spike(s[k]);
+#endif
 #if LEAN_EMP >= 0
       if (lastw[k] != NEVER && (n0 + w) - (int64_t)lastw[k] <= LEAN_EMP) sp = false;
 #endif

@@ -555,3 +555,53 @@ def test_group_without_threshold_never_spikes(lean):
     assert h.spike_count(g) == 0
     np.testing.assert_array_equal(h.get_state(g, 0, 300), x0 * 0.5 ** 20)
     h.close()
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("npt,delay,n,refr", [(1, 5, 700, False), (2, 3, 257, True), (4, 1, 2000, False),
+                                              (4, 12, 513, False), (1, 20, 1, True)])
+def test_lean_kernel_float_rings_and_sources(precision, npt, delay, n, refr):
+    """k_lean with two float rings and a packed count ring, driven by Poisson
+    sources (constant rates and a rate table) on k_lean, against the general
+    kernels (BM_TUNE_LEAN 0).  Weights are multiples of 2^-10, so their sums
+    are exact in any order: rasters and state equal bit for bit.  (4, 12) has
+    more ring words than k_lean keeps and runs the general kernel."""
+    from brian_amd._lib import NetHandle
+    out = []
+    for lean in (1, 0):
+        rng = np.random.default_rng(n + delay)
+        h = NetHandle(1e-4, precision)
+        p = h.add_poisson(300, 50.0 + 100.0 * rng.random(300), 3)
+        g = h.add_group(rng.random((3, n)))
+        A = np.array([[0.95, 0.03, -0.02], [0.0, 0.9, 0.0], [0.0, 0.0, 0.8]])
+        h.set_linear(g, A, np.array([0.02, 0.0, 0.0]))
+        h.set_threshold(g, 0, 0.9)
+        h.add_reset_op(g, 0, 0, 0.0)
+        if refr:
+            h.set_refractory(g, 21, 2e-3 - 0.5e-4)
+
+        def csr(ns, k):
+            return np.arange(ns + 1) * k, np.sort(rng.integers(0, n, (ns, k)), axis=1).ravel()
+
+        def weights(m):
+            return rng.integers(1, 300, m) / 1024.0
+        k = min(20, n)
+        ptr, col = csr(300, k)
+        h.add_connection(p, 0, 300, g, 0, n, 1, ptr, col, weights(len(col)), syn_delay=rng.integers(delay, delay + 9, len(col)),
+                         max_delay_steps=delay + 9)
+        ptr, col = csr(n, 3)
+        h.add_connection(g, 0, n, g, 0, n, 2, ptr, col, weights(len(col)), delay_steps=delay)
+        ptr, col = csr(300, 2)
+        h.add_connection(p, 0, 300, g, 0, n, 1, ptr, col, np.full(len(col), 0.125), delay_steps=delay + 1)
+        h.record(g, 1 << 18)
+        h.record(p, 1 << 18)
+        h.set_poisson_rates(p, 50, 500.0 * rng.random((40, 300)), True)
+        h.prepare(neurons_per_thread=npt)
+        h.set_tuning("lean", lean)
+        h.run(37)
+        h.run(300)
+        out.append([*h.get_spikes(g), *h.get_spikes(p), *[h.get_state(g, v, n) for v in range(3)]])
+        h.close()
+    assert len(out[0][0]) > 3 and len(out[0][2]) > 300
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
