@@ -24,6 +24,13 @@
 // step keeps a fast wavefront from overwriting a list still being read.
 // FP32 weights are accumulated with Kahan compensation; FP64 (check mode)
 // uses plain adds.
+//
+// Bound by the vector unit: a 1024 x 1000 FP32 step at 4 x 4 issues 70 VALU
+// instructions a wavefront, eight of them quarter-rate multiplies, which is 376 of
+// the 414 issue slots its four wavefronts a SIMD have.  93 of them took 0.96 us
+// a step; scalar lane masks for the spikes, one branch over a wavefront's four
+// slots, first list entries read ahead of the draws and variable indices known
+// at compile time make it 0.84.
 #include "common.hpp"
 #include "../../include/brianmi.h"
 
@@ -53,9 +60,13 @@ struct StdpBatchDev {
 template <typename T>
 __device__ inline T clipw(T x, T lo, T hi) { return x < lo ? lo : (x > hi ? hi : x); }
 
-template <typename T, int M, bool KAHAN, int NW, int NJ>
+// V010: the neuron's variables are those of a membrane potential 0 with a
+// threshold and a reset and a conductance 1 that the inputs add to, known at
+// compile time (else the indices are compared every step).
+template <typename T, int M, bool KAHAN, int NW, int NJ, bool V010>
 __global__ __launch_bounds__(64 * NW) void k_stdp_batch(const StdpBatchDev d, int64_t n0, int nsteps) {
 #pragma clang fp contract(off)
+  const int th_var = V010 ? 0 : d.th_var, tgt_var = V010 ? 1 : d.tgt_var, reset_var = V010 ? 0 : d.reset_var;
   const int inst = blockIdx.x;
   if (inst >= d.ninst) return;  // uniform over the workgroup
   const int lane = threadIdx.x & 63;
@@ -66,7 +77,7 @@ __global__ __launch_bounds__(64 * NW) void k_stdp_batch(const StdpBatchDev d, in
   T *wc = static_cast<T *>(d.wc) + (int64_t)inst * nin;
   T *ap = static_cast<T *>(d.apre) + (int64_t)inst * nin;
   __shared__ T sh_list[NW > 1 ? 2 * NW * 64 * NJ : 1];
-  __shared__ int sh_cnt[NW > 1 ? 2 * NW : 1];
+  __shared__ __align__(4) uint16_t sh_cnt[NW > 1 ? 2 * NW : 2];
   T rw[NJ], rc[NJ], ra[NJ];
   uint32_t key[NJ];
   bool valid[NJ];
@@ -101,16 +112,49 @@ __global__ __launch_bounds__(64 * NW) void k_stdp_batch(const StdpBatchDev d, in
   // The inputs' spikes of a step depend on nothing else in the step, so each
   // step computes the next step's while the other wavefronts' spike lists
   // are read from LDS (the hashes fill that wait instead of lengthening the
-  // chain from the barrier to the neuron update).
-  bool spk_next[NJ];
+  // chain from the barrier to the neuron update).  They are kept as one lane
+  // mask per slot in scalar registers: at 15 Hz a slot of 64 inputs spikes in
+  // one step of eleven, and all a slot's spikes cost (listing them, the pre
+  // updater) sits behind a scalar branch on its mask.  The draw is weyl_u32's,
+  // with its last round h ^= h >> 16, which leaves the upper half as it is,
+  // taken only where some lane's upper half could pass.
+  const uint32_t lim = (uint32_t)(d.thr - 1ull), lim_hi = lim | 0xFFFFu;   // spike iff u32 <= lim; thr 0: no input
+  unsigned long long on[NJ], next[NJ], next_any = 0ull;
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) spk_next[j] = valid[j] && (uint64_t)weyl_u32(key[j], (uint32_t)n0) < d.thr;
+  for (int j = 0; j < NJ; ++j) on[j] = d.thr == 0 ? 0ull : __ballot(valid[j]);
+  const auto draw = [&](uint32_t n) {
+    const uint32_t at = n * 0x9E3779B9u;
+    unsigned long long any = 0ull;
+    uint32_t hs[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      uint32_t h = key[j] + at;
+      h ^= h >> 16;
+      h *= 0x85EBCA6Bu;
+      h ^= h >> 13;
+      h *= 0xC2B2AE35u;
+      hs[j] = h;
+      next[j] = __ballot(h <= lim_hi) & on[j];
+      any |= next[j];
+    }
+    if (any != 0ull) {
+      any = 0ull;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        next[j] = __ballot((hs[j] ^ (hs[j] >> 16)) <= lim) & on[j];
+        any |= next[j];
+      }
+    }
+    next_any = any;
+  };
+  draw((uint32_t)n0);
   for (int st = 0; st < nsteps; ++st) {
     const uint32_t n = (uint32_t)(n0 + st);
     // ---- groups: inputs, neuron state update + threshold, trace decay
-    bool spk[NJ];
+    unsigned long long spk[NJ];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) spk[j] = spk_next[j];
+    for (int j = 0; j < NJ; ++j) spk[j] = next[j];
+    const unsigned long long any = next_any;    // some input of this wavefront spikes
     {
       T tmp[M];
 #pragma unroll
@@ -126,61 +170,82 @@ __global__ __launch_bounds__(64 * NW) void k_stdp_batch(const StdpBatchDev d, in
     T vth = s[0];
 #pragma unroll
     for (int r = 0; r < M; ++r)
-      if (r == d.th_var) vth = s[r];
+      if (r == th_var) vth = s[r];
     const bool post = vth > vt;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) ra[j] = dp * ra[j] + (T)0;
-    apost = dm * apost + (T)0;
+    for (int j = 0; j < NJ; ++j) ra[j] = dp * ra[j];
+    apost = dm * apost;
     // ---- connections: propagation in ascending input order
     T x = s[0];
 #pragma unroll
     for (int r = 0; r < M; ++r)
-      if (r == d.tgt_var) x = s[r];
+      if (r == tgt_var) x = s[r];
     if constexpr (NW == 1) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        unsigned long long mask = __ballot(spk[j]);
+        unsigned long long mask = spk[j];
         while (mask) {
           const int l = __ffsll((long long)mask) - 1;
           mask &= mask - 1ull;
           x = x + __shfl(rw[j], l);
         }
       }
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) spk_next[j] = valid[j] && (uint64_t)weyl_u32(key[j], n + 1u) < d.thr;
+      draw(n + 1u);
     } else {
       const int b = st & 1;
       T *list = sh_list + (b * NW + wv) * 64 * NJ;
       int cnt = 0;
+      if (any != 0ull) {
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const unsigned long long mask = __ballot(spk[j]);
-        const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-        if (spk[j]) list[cnt + below] = rw[j];
-        cnt += __popcll(mask);
+        for (int j = 0; j < NJ; ++j) {
+          const unsigned long long mask = spk[j];
+          if (mask == 0ull) continue;
+          const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+          if ((mask >> lane) & 1ull) list[cnt + below] = rw[j];
+          cnt += __popcll(mask);
+        }
+      } else if (lane == 0) {
+        list[0] = (T)0;           // an empty list adds nothing
       }
-      if (lane == 0) sh_cnt[b * NW + wv] = cnt;
+      if (lane == 0) sh_cnt[b * NW + wv] = (uint16_t)cnt;
       __syncthreads();
-      int cnts[NW];
+      // the counts, two to a word, and every list's first entry are read
+      // together (a list has more than one in one step of twenty), and the
+      // next step's draws fill the wait
+      uint32_t words[NW / 2];
+      T head[NW];
 #pragma unroll
-      for (int v = 0; v < NW; ++v) cnts[v] = sh_cnt[b * NW + v];
+      for (int v = 0; v < NW / 2; ++v) words[v] = reinterpret_cast<const uint32_t *>(sh_cnt + b * NW)[v];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) spk_next[j] = valid[j] && (uint64_t)weyl_u32(key[j], n + 1u) < d.thr;
+      for (int v = 0; v < NW; ++v) head[v] = sh_list[(b * NW + v) * 64 * NJ];
+      draw(n + 1u);
+      uint32_t all = 0u;
 #pragma unroll
-      for (int v = 0; v < NW; ++v) {
-        const int c = __builtin_amdgcn_readfirstlane(cnts[v]);
-        const T *lv = sh_list + (b * NW + v) * 64 * NJ;
-        for (int k = 0; k < c; ++k) x = x + lv[k];
+      for (int v = 0; v < NW / 2; ++v) {
+        words[v] = __builtin_amdgcn_readfirstlane(words[v]);
+        all |= words[v];
+      }
+      if ((all & 0xFFFEFFFEu) == 0u) {
+#pragma unroll
+        for (int v = 0; v < NW; ++v) x = x + head[v];
+      } else {
+#pragma unroll
+        for (int v = 0; v < NW; ++v) {
+          const int c = (int)((words[v / 2] >> (16 * (v & 1))) & 0xFFFFu);
+          const T *lv = sh_list + (b * NW + v) * 64 * NJ;
+          for (int k = 0; k < c; ++k) x = x + lv[k];
+        }
       }
     }
 #pragma unroll
     for (int r = 0; r < M; ++r)
-      if (r == d.tgt_var) s[r] = x;
+      if (r == tgt_var) s[r] = x;
     // ---- pre updater
+    if (any != 0ull)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-      if (!spk[j]) continue;
+      if (spk[j] == 0ull || !((spk[j] >> lane) & 1ull)) continue;
       ra[j] = (d.interactions == 0 || d.interactions == 3) ? ra[j] + Ap : Ap;
       if (d.update == 0 && KAHAN) {
         const T y = apost - rc[j];
@@ -226,7 +291,7 @@ __global__ __launch_bounds__(64 * NW) void k_stdp_batch(const StdpBatchDev d, in
       // ---- reset
 #pragma unroll
       for (int r = 0; r < M; ++r)
-        if (r == d.reset_var) s[r] = vr;
+        if (r == reset_var) s[r] = vr;
       if (threadIdx.x == 0 && d.raster != nullptr) {
         const unsigned long long pos = atomicAdd(d.raster_count, 1ull);
         if (pos < (unsigned long long)d.raster_cap) d.raster[pos] = ((uint64_t)n << 32) | (uint64_t)inst;
@@ -267,12 +332,12 @@ inline void stdp_default_layout(int nin, int *nw, int *nj) {
   *nw = w;
 }
 
-template <typename T, int M, bool KAHAN>
+template <typename T, int M, bool KAHAN, bool V010>
 void launch_stdp_m(const StdpBatchDev &d, int nw, int nj, int64_t n0, int nsteps, hipStream_t st) {
   const dim3 g(d.ninst);
 #define BM_SB(NW_, NJ_)                                                                        \
   if (nw == NW_ && nj == NJ_) {                                                                \
-    hipLaunchKernelGGL((k_stdp_batch<T, M, KAHAN, NW_, NJ_>), g, dim3(64 * NW_), 0, st, d, n0, \
+    hipLaunchKernelGGL((k_stdp_batch<T, M, KAHAN, NW_, NJ_, V010>), g, dim3(64 * NW_), 0, st, d, n0, \
                        nsteps);                                                                \
     return;                                                                                    \
   }
@@ -286,10 +351,15 @@ void launch_stdp_m(const StdpBatchDev &d, int nw, int nj, int64_t n0, int nsteps
 template <typename T, bool KAHAN>
 void launch_stdp_batch(const StdpBatchDev &d, int nw, int nj, int64_t n0, int nsteps, hipStream_t st) {
   switch (d.M) {
-    case 1: launch_stdp_m<T, 1, KAHAN>(d, nw, nj, n0, nsteps, st); break;
-    case 2: launch_stdp_m<T, 2, KAHAN>(d, nw, nj, n0, nsteps, st); break;
-    case 3: launch_stdp_m<T, 3, KAHAN>(d, nw, nj, n0, nsteps, st); break;
-    default: launch_stdp_m<T, 4, KAHAN>(d, nw, nj, n0, nsteps, st); break;
+    case 1: launch_stdp_m<T, 1, KAHAN, false>(d, nw, nj, n0, nsteps, st); break;
+    case 2:
+      if (d.th_var == 0 && d.tgt_var == 1 && d.reset_var == 0)
+        launch_stdp_m<T, 2, KAHAN, true>(d, nw, nj, n0, nsteps, st);
+      else
+        launch_stdp_m<T, 2, KAHAN, false>(d, nw, nj, n0, nsteps, st);
+      break;
+    case 3: launch_stdp_m<T, 3, KAHAN, false>(d, nw, nj, n0, nsteps, st); break;
+    default: launch_stdp_m<T, 4, KAHAN, false>(d, nw, nj, n0, nsteps, st); break;
   }
 }
 

@@ -148,3 +148,35 @@ def test_stdp_batch_c3_fp32_vs_fp64_histogram():
           f"post spikes {len(res[32][1][0])} vs {len(res[64][1][0])}")
     assert tv < 0.05
     print("FP64 final weight histogram (20 bins of gmax/20):", np.round(h64, 4).tolist())
+
+
+@pytest.mark.parametrize("rate", [0.0, 15.0, 3000.0, 10000.0])
+@pytest.mark.parametrize("precision", [32, 64])
+def test_stdp_batch_variable_order_and_layouts(precision, rate):
+    """The neuron's two variables in either order (the order of the reference's
+    example is compiled in, others are compared every step) and every layout,
+    from no input spikes to one per input and step: equal bit for bit (a sum of
+    two products has the same bits in either order)."""
+    A, C, dp, dm, Ap, Am = stdp_consts()
+    ninst, nin, steps = 3, 130, 300
+    w0 = np.random.default_rng(1).random((ninst, nin)) * gmax
+    S0 = np.zeros((ninst, 2))
+    S0[:, 0] = vr
+    out = []
+    for swap in (False, True):
+        for nw, nj in ((0, 0), (4, 1), (2, 2), (8, 1), (16, 1), (1, 4), (2, 4)):
+            if swap and (nw, nj) not in ((0, 0), (4, 1)):
+                continue
+            o = [1, 0] if swap else [0, 1]
+            h = StdpBatchHandle(precision, DT, ninst, nin, A[np.ix_(o, o)], C[o], S0[:, o], o.index(0), vt, o.index(0),
+                                vr, o.index(1), w0, rate, 9, dp, dm, Ap, Am, 0.0, gmax)
+            h.set_layout(nw, nj)
+            h.run(steps)
+            h.run(7)
+            out.append([h.weights(), h.a_pre(), h.a_post(), h.state()[:, o], *h.spikes()])
+            h.close()
+    assert (len(out[0][4]) > 0) == (rate > 1000.0)
+    assert (out[0][1].max() > 0) == (rate > 0)
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            np.testing.assert_array_equal(a, b)
