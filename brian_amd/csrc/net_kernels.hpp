@@ -26,6 +26,11 @@ namespace bm {
 // ------------------------------------------------------------------ helpers
 __device__ inline int lane_id() { return __lane_id(); }
 
+// Ring slot of step n (n >= 0).  Steps are below 2^31, as the 32-bit last
+// spike steps and rasters need: a 32-bit remainder instead of a 64-bit one,
+// whose 100 or so instructions each launch waited for before its first ring load.
+__device__ inline int step_mod(int64_t n, int D) { return (int)((uint32_t)n % (uint32_t)D); }
+
 template <typename T>
 __device__ inline T dev_exp(T x) { return exp(x); }
 template <typename T>
@@ -392,7 +397,7 @@ __device__ inline void propagate_waves(const GroupDev &g, const uint16_t *sh_lis
       const OutDev &od = g.outs[o];
       const int64_t r = (int64_t)i - od.src_off;
       if (r < 0 || r >= od.src_n) continue;
-      const int base_slot = (int)(n % od.D);
+      const int base_slot = step_mod(n, od.D);
       const int64_t lo = od.row_ptr[r], hi = od.row_ptr[r + 1];
       const int pbits = od.nch * od.bits;
       for (int64_t q = lo + sl; q < hi; q += rs) {
@@ -442,7 +447,7 @@ __device__ inline void propagate_block(const GroupDev &g, const uint16_t *sh_lis
           lo = od.row_ptr[r];
           len = (int)(od.row_ptr[r + 1] - lo);
         }
-        sb = (int)(n % od.D);
+        sb = step_mod(n, od.D);
       }
       int total = 0;
       const int off = block_exclusive_scan(len, tid, sh_wsum, &total);
@@ -567,8 +572,7 @@ __global__ __launch_bounds__(BLOCK) void k_sweep(const GroupDev g, const int64_t
   }
   const int nsteps = tail_only ? 1 : W;
   // ring slot of the tail at window offset w is (n0 - 1 + w) mod D
-  int slot0 = (int)((n0 - 1) % D);
-  if (slot0 < 0) slot0 += D;
+  const int slot0 = step_mod(n0 + D - 1, D);
 
   for (int w0 = 0; w0 < nsteps; w0 += PF) {
     uint32_t cw[PF][K];
@@ -1000,7 +1004,7 @@ __global__ __launch_bounds__(BLOCK) void k_sweep(const GroupDev g, const int64_t
     }
     // ---------------- spike history for STDP (only with W == 1)
     if (g.hist != nullptr) {
-      const int64_t hs = n0 % g.H;
+      const int64_t hs = step_mod(n0, g.H);
       if (tid == 0) sh_hbase = atomicAdd(&g.hist_count[hs], (unsigned int)nsp);
       __syncthreads();
       for (int p = tid; p < nsp; p += BLOCK)
@@ -1105,7 +1109,7 @@ __global__ __launch_bounds__(BLOCK) void k_generator(const GroupDev g, const int
         int d = od.hom_delay;
         if (od.dly_bytes == 1) d = static_cast<const uint8_t *>(od.dly)[qq];
         else if (od.dly_bytes == 2) d = static_cast<const uint16_t *>(od.dly)[qq];
-        const int64_t sl = (n + d) % od.D;
+        const int64_t sl = step_mod(n + d, od.D);
         unsigned char *slot = static_cast<unsigned char *>(od.ring) + sl * od.slot_bytes;
         if (od.kind == RING_COUNT) {
           const int64_t pos = tj * (od.nch * od.bits) + od.ch * od.bits;

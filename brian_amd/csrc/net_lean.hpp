@@ -101,8 +101,7 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
   uint32_t cw[LEAN_WMAX][K][NR];
   T fw[LEAN_WMAX][K][NR];
 #if LEAN_NRING > 0
-  int slot0 = (int)((n0 - 1) % g.D);
-  if (slot0 < 0) slot0 += g.D;
+  const int slot0 = step_mod(n0 + g.D - 1, g.D);
 #pragma unroll
   for (int u = 0; u < LEAN_WMAX; ++u) {
 #pragma unroll
@@ -257,7 +256,7 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
     }
     // spike history for STDP (networks with STDP run one step per launch)
     if (g.hist != nullptr) {
-      const int64_t hs = n0 % g.H;
+      const int64_t hs = step_mod(n0, g.H);
       if (tid == 0) sh_hbase = atomicAdd(&g.hist_count[hs], (unsigned int)nsp);
       __syncthreads();
       for (int p = tid; p < nsp; p += BLOCK)
