@@ -1870,8 +1870,9 @@ void prepare(bm_net *net, int window, int K, int use_graph) {
     net->lates.push_back(lm);
   }
   check_launch_shapes(net);
-  ensure_jit(net);
-  (void)ensure_small(net);
+  // a small network compiles its own kernel; its groups' sweeps, which only runs
+  // of a few steps take, at the first such run
+  if (!ensure_small(net)) ensure_jit(net);
   net->d_base.alloc(8);
   int64_t zero = 0;
   BM_HIP(hipMemcpyAsync(net->d_base.p, &zero, 8, hipMemcpyHostToDevice, net->stream));
