@@ -689,9 +689,8 @@ def bench_stdp(args):
                            "weights and traces in registers)",
                     steps_per_launch=steps_per_launch, avg_launch_us=avg_launch_s * 1e6,
                     alg_bytes_per_launch=alg_bytes, launches_timed=launches,
-                    note="register-resident weights: HBM is not the bound; the latency of each "
-                         "step's chain (hashes, ballot, LDS spike lists, barrier, fold, neuron "
-                         "update) at four wavefronts per SIMD is")
+                    note="register-resident weights: HBM is not the bound; vector "
+                         "instruction issue (the input hashes foremost) is")
     check = None
     if 64 in res:
         bins = np.linspace(0, d["gmax"], 21)
@@ -906,7 +905,7 @@ def bench_mlp(args):
                                f"{epochs} epochs, Adam", "pairs": n, "epochs": epochs, "final_loss": loss},
         "roofline": {"bound": "mfma", "achieved": tflops, "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": tflops / BF16_PEAK_TFLOPS, "traffic": None,
-                     "kernel": "k_mlp_rows + k_mlp_wgrad + k_mlp_adam (one training step)",
+                     "kernel": "k_mlp_rows + k_mlp_wgrad (one training step)",
                      "flops_per_sample": MLP_FLOPS_SAMPLE},
         "cpu_baseline": None,
     }
