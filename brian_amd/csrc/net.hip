@@ -457,10 +457,13 @@ std::string jit_list(const std::vector<int> &v) {
   return o.str();
 }
 
-// A double as a C++ hexadecimal literal (exact), cast to float for FP32.
+// A double as a C++ hexadecimal literal (exact), cast to float for FP32; an
+// infinite threshold (a group that never spikes) or a NaN has no literal.
 std::string lit(double v, bool f32) {
   char buf[64];
-  std::snprintf(buf, sizeof buf, "%a", v);
+  if (std::isnan(v)) std::snprintf(buf, sizeof buf, "__builtin_nan(\"\")");
+  else if (std::isinf(v)) std::snprintf(buf, sizeof buf, "%s__builtin_inf()", v < 0 ? "-" : "");
+  else std::snprintf(buf, sizeof buf, "%a", v);
   return f32 ? std::string("(float)(") + buf + ")" : std::string("(") + buf + ")";
 }
 

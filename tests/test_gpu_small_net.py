@@ -9,6 +9,7 @@ import pytest
 
 from brian_amd import workloads as W
 from brian_amd._lib import NetHandle
+from brian_amd.equations import Equations
 from tests.netbuild import cuba_propagator
 
 pytestmark = pytest.mark.gpu
@@ -161,5 +162,39 @@ def test_long_run_and_rate_changes():
         out.append(read(h))
         h.close()
     assert len(out[0][0]) > 20
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("vt", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("steps", [3, 40])     # windowed kernels, one workgroup
+@pytest.mark.parametrize("kind", ["counts", "weights", "program"])
+def test_constants_without_a_literal(kind, steps, vt):
+    """Thresholds and reset values that are infinite or NaN, against the kernels
+    that read them from tables (specialize 0)."""
+    out = []
+    for specialize in (1, 0):
+        n = 70
+        h = NetHandle(DT, 64)
+        g = h.add_group(np.random.default_rng(3).random((2, n)))
+        if kind == "program":
+            code, consts, nregs = Equations("dv/dt = (b - v)/(10*ms) : 1\ndw/dt = -w*w/(20*ms) : 1",
+                                            b=vt).compile_program()
+            h.set_program(g, 1, nregs, code, consts)
+            h.set_threshold(g, 1, 0.5)
+            h.add_reset_op(g, 1, 0, 0.9)
+        else:
+            h.set_linear(g, np.diag([0.99, 0.98]), np.zeros(2))
+            h.set_threshold(g, 0, vt)
+            h.add_reset_op(g, 1, 0, -vt)
+        w = np.full(n, 0.01) if kind == "counts" else 0.01 * np.arange(n)
+        h.add_connection(g, 0, n, g, 0, n, 0, np.arange(n + 1), np.arange(n), w)
+        h.record(g, 1 << 14)
+        h.prepare()
+        h.set_tuning("specialize", specialize)
+        h.run(steps)
+        out.append([*h.get_spikes(g), h.get_state(g, 0, n), h.get_state(g, 1, n)])
+        h.close()
+    assert len(out[0][0]) == (0 if kind != "program" and not vt < 0 else len(out[1][0]))
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
