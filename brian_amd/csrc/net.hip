@@ -194,7 +194,8 @@ struct bm_net {
   JitKernel small;        // the whole network in one workgroup (net_small.hpp)
   DevBuf small_d;         // its descriptors, and what they were last copied from
   std::vector<unsigned char> small_h;
-  DevBuf raster_work;     // buffers of the raster sort, as large as the largest raster read so far
+  DevBuf raster_work;     // buffers of the raster sort, as large as the largest raster read so far,
+  std::mutex raster_mu;   // held by the reading thread that uses them
   DevBuf hist_ptrs_d, hist_H_d;
   int nhist = 0;
   std::vector<LateModDev> lates;   // modulated Connections with a homogeneous delay
@@ -3038,6 +3039,7 @@ int bm_net_get_spikes(bm_net *net, int gid, int32_t *steps, int32_t *idx, int64_
     // sorted on the device, unless its buffers do not fit there
     const size_t want = raster_sort_bytes(c, g.raster_first, net->step, g.N);
     bool fits = c < (int64_t(1) << 31);
+    std::unique_lock<std::mutex> lk(net->raster_mu);
     if (fits && net->raster_work.bytes < want) {
       try {
         net->raster_work.alloc(want);
@@ -3055,6 +3057,7 @@ int bm_net_get_spikes(bm_net *net, int gid, int32_t *steps, int32_t *idx, int64_
       BM_HIP(hipStreamSynchronize(net->stream));
       return;
     }
+    lk.unlock();
     std::vector<uint64_t> tmp = fetch_raster(net, g, cs, c, nullptr);
     std::sort(tmp.begin(), tmp.end());
     for (size_t q = 0; q < tmp.size(); ++q) {

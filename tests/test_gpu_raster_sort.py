@@ -2,6 +2,8 @@
 index), repeats kept, at the sizes where the path changes (one workgroup's
 LDS, one tile of the radix sort, several tiles, 64-bit keys), against numpy's
 sort of the generator's table."""
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -35,4 +37,24 @@ def test_raster_is_sorted(n, N, steps):
     b = h.get_spikes(g)
     np.testing.assert_array_equal(b[0], s)
     np.testing.assert_array_equal(b[1], i)
+    h.close()
+
+
+def test_rasters_read_by_several_threads():
+    rng = np.random.default_rng(5)
+    h = NetHandle(1e-4, 32)
+    want = {}
+    for n in (500, 20000, 60000):
+        s, i = np.sort(rng.integers(0, 200, n)), rng.integers(0, 3000, n)
+        order = np.lexsort((i, s))
+        g = h.add_generator(3000, s[order], i[order])
+        h.record(g, n * 64)
+        want[g] = (s[order], i[order])
+    h.prepare()
+    h.run(200)
+    with ThreadPoolExecutor(6) as pool:
+        reads = [(g, pool.submit(h.get_spikes, g)) for _ in range(8) for g in want]
+        for g, r in reads:
+            np.testing.assert_array_equal(r.result()[0], want[g][0])
+            np.testing.assert_array_equal(r.result()[1], want[g][1])
     h.close()
