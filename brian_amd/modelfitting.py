@@ -306,14 +306,14 @@ class FitEngine:
             self._P = np.zeros((max(len(self.param_names), 1), self.ncand))
         P = self._P
         for k, p in enumerate(self.param_names):
-            P[k] = params[p]
+            P[k] = np.broadcast_to(np.asarray(params[p], dtype=np.float64), (self.ncand,))
         S = None
         if init_state is not None:
             if self._S is None:
                 self._S = np.zeros((len(self.state_names), self.ncand))
             S = self._S
             for k, v in enumerate(self.state_names):
-                S[k] = init_state.get(v, 0.0)
+                S[k] = np.broadcast_to(np.asarray(init_state.get(v, 0.0), dtype=np.float64), (self.ncand,))
         r = None if refractory_steps is None else np.ascontiguousarray(
             np.broadcast_to(refractory_steps, (self.ncand,)), dtype=np.int32)
         d = None if delay_steps is None else np.ascontiguousarray(

@@ -197,3 +197,20 @@ def test_device_ou_input_matches_oracle(precision):
     for j in range(n):
         np.testing.assert_array_equal(trains[j], want[j])
     eng.close()
+
+
+@pytest.mark.parametrize("bad", [np.zeros((1, 8)), np.zeros(7), np.zeros((8, 1))])
+def test_candidate_values_of_another_shape_are_refused(bad):
+    """The arrays kept between candidate sets take what broadcasting to one
+    value per candidate does, and a refused set leaves nothing behind."""
+    n = 8
+    eng = FitEngine(fit_eqs(), W.FIT_THRESHOLD, W.FIT_RESET, np.ones((1, 100)), [np.zeros(0)], np.zeros(n, int), DT,
+                    40, precision=64)
+    good = {k: 1.0 + np.arange(n) for k in eng.param_names}
+    eng.set_candidates(good)
+    with pytest.raises(ValueError):
+        eng.set_candidates({**good, eng.param_names[-1]: bad})
+    with pytest.raises(ValueError):
+        eng.set_candidates(good, init_state={eng.state_names[0]: bad})
+    eng.set_candidates({k: 2.0 for k in eng.param_names}, init_state={})
+    eng.close()
