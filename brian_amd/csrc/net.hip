@@ -1114,7 +1114,7 @@ std::string small_source(bm_net *net) {
     << "  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;\n"
     << "  if (tid < 2 * SMALL_GROUPS) cnt[tid] = 0;\n";
   for (int gi = 0; gi < ng; ++gi)
-    d << "  SmallRegs<SG" << gi << "> r" << gi << ";\n  SmallRaster rr" << gi << " = {0, (int)(n0 & 31)};\n  const int D" << gi
+    d << "  SmallRegs<SG" << gi << "> r" << gi << ";\n  SmallRaster rr" << gi << " = {0};\n  const int D" << gi
       << " = gd[" << gi << "].D, N" << gi << " = (int)gd[" << gi << "].N;\n  int sl" << gi << " = (int)(n0 % D" << gi
       << ");\n  small_load<SG" << gi << ">(gd[" << gi << "], r" << gi << ", sm, sn, tid);\n";
   for (size_t s = 0; s < net->stdps.size(); ++s)

@@ -287,14 +287,20 @@ __device__ inline void small_traces(const StdpDev &sd, unsigned char *sm, const 
 }
 
 // Raster of a group: one wavefront stages entries in LDS and appends
-// SMALL_RASTER of them at a time to the append regions in turn (one workgroup
-// fills them all; a region by its block index would take the whole raster).
+// SMALL_RASTER of them at a time to the append region with the fewest (one
+// workgroup fills them all; a region by its block index would take the whole
+// raster, and one by the step most of it where runs are of 32 steps).
 struct SmallRaster {
-  int cnt, region;
+  int cnt;
 };
 __device__ inline void small_raster_flush(const GroupDev &g, const unsigned long long *buf, SmallRaster &rr, int lane) {
   if (rr.cnt == 0) return;
-  const int shard = rr.region++ & (RSHARD - 1);
+  unsigned long long least = ~0ull;
+  if (lane < RSHARD)
+    least = __hip_atomic_load(g.raster_count + lane * RSTRIDE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * RSHARD + lane;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) least = min(least, (unsigned long long)__shfl_xor(least, o));
+  const int shard = (int)(least % RSHARD);
   unsigned long long at = 0;
   if (lane == 0) at = atomicAdd(g.raster_count + shard * RSTRIDE, (unsigned long long)rr.cnt);
   at = __shfl(at, 0);

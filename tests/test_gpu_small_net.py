@@ -198,3 +198,23 @@ def test_constants_without_a_literal(kind, steps, vt):
     assert len(out[0][0]) == (0 if kind != "program" and not vt < 0 else len(out[1][0]))
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+def test_raster_regions_fill_evenly():
+    """Runs of as many steps as there are append regions: the raster still
+    holds the capacity asked for."""
+    n, runs = 3000, 64
+
+    def build():
+        h = NetHandle(DT, 64)
+        g = h.add_group(np.random.default_rng(1).random((1, n)))
+        h.set_linear(g, np.eye(1), np.array([1 / 150]))
+        h.set_threshold(g, 0, 1.0)
+        h.add_reset_op(g, 0, 0, 0.0)
+        h.add_connection(g, 0, 1, g, 0, n, 0, np.array([0, 1]), np.array([0]), np.array([1e-3]))
+        h.record(g, n * 32 * runs // 140)
+        h.prepare()
+        return h, lambda h: [*h.get_spikes(g), h.get_state(g, 0, n)]
+
+    out = _both(build, [32] * runs)
+    assert len(out[0]) > n * 32 * runs // 160
