@@ -189,6 +189,7 @@ struct bm_net {
   int defer_req = 0;      // BM_TUNE_DEFER before prepare
   int defer_W = 0;        // largest window with deferred propagation, 0 = off
   int64_t step = 0;       // next step to run
+  int route = 0;          // how the last run was launched (BM_TUNE_ROUTE)
   hipStream_t stream = nullptr;
   DevBuf d_base;          // int64 device step base
   JitKernel small;        // the whole network in one workgroup (net_small.hpp)
@@ -769,19 +770,24 @@ void ensure_jit(bm_net *net) {
 
 // ---- persistent launches for batches of independent networks (k_persist)
 // Three workgroup shapes.  A batch of no more networks than there are compute
-// units runs each on the widest: the networks have a unit each either way, and
-// all of them are one launch on the handle's stream.  (Three launches on three
-// streams run at once only where the runtime gives the streams hardware queues
-// of their own: 256 networks of 500 to 20,000 neurons took 19.3 ms for 1000 steps
-// and their raster and state with two of the launches one after the other, 14.1
-// with one launch.)  In a
-// larger batch a network runs on the smallest shape that holds it (persist_kmax
-// neurons per thread), so that mid-size and small networks run two or four
-// workgroups to a compute unit and one network's memory latency overlaps
+// units is one launch of one shape on the handle's stream: the networks have a
+// unit each either way.  (Three launches on three streams run at once only where
+// the runtime gives the streams hardware queues of their own: 256 networks of 500
+// to 20,000 neurons took 19.3 ms for 1000 steps and their raster and state with
+// two of the launches one after the other, 14.1 with one launch.)  The shape is
+// the widest unless the largest network has at most PERSIST_NARROW neurons, for
+// which the barrier over 16 wavefronts costs more than their work saves: us a
+// step with the widest and the narrowest shape, FP32, 64 networks of 100 neurons
+// 1.36 and 0.97, of 250 1.68 and 1.32, of 500 1.96 and 1.79, of 600 2.06 and 2.18,
+// of 1000 2.34 and 2.50 (FP64: 500 2.18 and 2.11, 600 2.31 and 2.67).
+// In a larger batch a network runs on the smallest shape that holds it
+// (persist_kmax neurons per thread), so that mid-size and small networks run two
+// or four workgroups to a compute unit and one network's memory latency overlaps
 // another's work.
 constexpr int PERSIST_TIERS = 3;
 constexpr int PERSIST_TIER_BLOCK[PERSIST_TIERS] = {1024, 512, 256};
 constexpr int PERSIST_BLOCK = 1024;  // the largest shape
+constexpr int64_t PERSIST_NARROW = 512;
 // neurons per thread of the largest body of k_persist (net_persist.hpp):
 // 20 in FP32, the last 4 slots' state in LDS (models of up to 3 variables),
 // 16 for larger FP32 models, 8 in FP64
@@ -791,7 +797,7 @@ int persist_kmax(const bm_net *net, const HostGroup &g) {
 }
 // the shape of a network of np neurons
 int persist_tier(const bm_net *net, const HostGroup &g, int64_t np) {
-  if ((int)g.part_off.size() - 1 <= net->compute_units) return 0;
+  if ((int)g.part_off.size() - 1 <= net->compute_units) return g.part_max > PERSIST_NARROW ? 0 : PERSIST_TIERS - 1;
   const int64_t K = persist_kmax(net, g);
   return np > 512 * K ? 0 : (np > 256 * K ? 1 : 2);
 }
@@ -951,6 +957,9 @@ void run_persist(bm_net *net, int64_t nsteps) {
                                      (unsigned)persist_shmem(net, g, block), st, args, nullptr));
         BM_HIP(hipGetLastError());
       };
+      // the largest network's shape
+      for (int t = PERSIST_TIERS - 1; t >= 0; --t)
+        if (first[t + 1] > first[t]) net->route = PERSIST_TIER_BLOCK[t];
       // the shapes in use run at once: the first on the handle's stream, the
       // others on streams of their own that join it afterwards
       int used[PERSIST_TIERS], nused = 0;
@@ -1915,9 +1924,11 @@ void run(bm_net *net, int64_t nsteps) {
     return;
   }
   if (nsteps >= SMALL_MIN_STEPS && !net->profiling && ensure_small(net)) {
+    net->route = BM_ROUTE_ONE_WORKGROUP;
     run_small(net, nsteps);
     return;
   }
+  net->route = BM_ROUTE_WINDOWS;
   ensure_jit(net);
   const int W = net->W;
   int64_t done = 0;
@@ -2914,6 +2925,7 @@ int bm_net_get_tuning(bm_net *net, int key, int *value) {
       case BM_TUNE_PERSIST: *value = net->persist ? 1 : 0; break;
       case BM_TUNE_PERSIST_CHUNK: *value = net->persist_chunk; break;
       case BM_TUNE_PERSIST_QUEUE: *value = net->persist_queue; break;
+      case BM_TUNE_ROUTE: *value = net->route; break;
       default: throw Error(BM_EINVAL, "unknown tuning key");
     }
   });

@@ -342,8 +342,10 @@ int bm_net_set_partition(bm_net *net, int gid, int nparts, const int64_t *offset
  *                              launch per group in which every network of the
  *                              group's partition (bm_net_set_partition) is
  *                              advanced by one workgroup (1024, 512 or 256
- *                              threads, the smallest that holds it) through
- *                              all the run's steps, state in registers, one
+ *                              threads: the smallest that holds it where there
+ *                              are more networks than compute units, else 256
+ *                              for networks of at most 512 neurons and 1024 for
+ *                              larger) through all the run's steps, state in registers, one
  *                              workgroup barrier per step.  Needs lean groups with count
  *                              rings, connections within a group, delays of
  *                              at least one step, no STDP, networks of at
@@ -357,7 +359,12 @@ int bm_net_set_partition(bm_net *net, int gid, int nparts, const int64_t *offset
  *                              queue is full is delivered through the count
  *                              ring instead, so results never depend on it;
  *                              the queues take D x N x value / 16 x 4 bytes,
- *                              allocated at the first persistent run */
+ *                              allocated at the first persistent run
+ *   BM_TUNE_ROUTE              (get only) how the last run was launched: 0 no run
+ *                              yet, BM_ROUTE_WINDOWS (a launch per group and
+ *                              window), BM_ROUTE_ONE_WORKGROUP (the whole network
+ *                              in one), or the threads of the largest network's
+ *                              workgroup in a persistent launch */
 enum {
   BM_TUNE_WINDOW = 1,
   BM_TUNE_NEURONS_PER_THREAD = 2,
@@ -372,8 +379,10 @@ enum {
   BM_TUNE_LEAN = 11,
   BM_TUNE_PERSIST = 12,
   BM_TUNE_PERSIST_CHUNK = 13,
-  BM_TUNE_PERSIST_QUEUE = 14
+  BM_TUNE_PERSIST_QUEUE = 14,
+  BM_TUNE_ROUTE = 15
 };
+enum { BM_ROUTE_WINDOWS = 1, BM_ROUTE_ONE_WORKGROUP = 2 };
 int bm_net_set_tuning(bm_net *net, int key, int value);
 int bm_net_get_tuning(bm_net *net, int key, int *value);
 

@@ -74,7 +74,7 @@ def test_persist_shape_boundaries(prec, more):
     """Networks at the edges of the three workgroup shapes (20 neurons per
     thread in FP32, 8 in FP64: 256, 512, 1024 threads), networks smaller
     than a wavefront, and empty runs between the chunks; alone (every network
-    on the widest shape) and with more networks than compute units (each on
+    on the largest one's shape) and with more networks than compute units (each on
     the smallest shape that holds it)."""
     K = 20 if prec == 32 else 8
     sizes = [1024 * K, 512 * K + 1, 512 * K, 256 * K + 1, 256 * K, 1, 7, 63, 64, 65, 256, 257, 1000] + [30] * more
@@ -88,6 +88,29 @@ def test_persist_shape_boundaries(prec, more):
     np.testing.assert_array_equal(pi, wi)
     for v in range(3):
         np.testing.assert_array_equal(pst[v], wst[v])
+
+
+@pytest.mark.parametrize("prec", [32, 64])
+@pytest.mark.parametrize("sizes,threads", [([512, 1, 300], 256), ([100] * 40, 256), ([513, 40], 1024),
+                                           ([60] * 300, 256), ([600] * 300, 256)])
+def test_persist_shape_of_few_networks(sizes, threads, prec):
+    """At most as many networks as compute units: networks of up to 512
+    neurons run on the narrowest workgroup, larger ones on the widest; more
+    networks each on the smallest that holds them."""
+    d = W.uneven_batch(seed=23, sizes=sizes, p=0.2)
+    out = []
+    for persist in (False, True):
+        h, g, _, _ = device_uneven(d, precision=prec)
+        if persist:
+            h.set_tuning("persist", 1)
+        assert h.get_tuning("route") == 0
+        h.run(400)
+        assert h.get_tuning("route") == (threads if persist else 1)
+        out.append([*h.get_spikes(g), *[h.get_state(g, v, d["N"]) for v in range(3)]])
+        h.close()
+    assert len(out[0][0]) > 50
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
 
 
 def test_persist_raster_overflow_reported():
