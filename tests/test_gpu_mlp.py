@@ -79,6 +79,56 @@ def test_mlp_widths_match_oracle(nin, nh, nu, B):
     m.close()
 
 
+@pytest.mark.parametrize("nin,nh,nu,B", [(17, 64, 2, 256), (40, 128, 4, 512), (90, 192, 8, 256), (256, 64, 16, 256),
+                                         (64, 256, 4, 1024), (90, 256, 3, 512)])
+def test_mlp_adam_steps(nin, nh, nu, B):
+    """Adam in the weight-gradient kernel, at every hidden width and with
+    inputs that are not a multiple of 32: four steps on one batch (the shuffle
+    only reorders its rows) against Adam in FP64 over the gradients that the
+    handle gives before each step, which the tests above hold to the oracle.
+
+    A row order changes a gradient element by under 2^-24 sqrt(B) of the terms
+    it sums, 1e-6 of the largest element; an element of at least 1e-3 of that
+    moves by 1e-3 of itself, and its update of at most lr by a few 1e-3 lr: 0.02
+    lr over four steps.  A smaller element may take the other sign (2 lr a
+    step), one without a gradient stays where it is.
+
+    After the steps a handle made anew from the parameters gives the same bits:
+    the BF16 copies of the weights, in both layouts, are those of the
+    parameters."""
+    rng = np.random.default_rng(nin * nh)
+    lr, steps = 1e-3, 4
+    p0 = L.init_params(nin, nh, nu, seed=4)
+    p0 = (p0 + 0.05 * rng.standard_normal(len(p0))).astype(np.float32)
+    X = rng.standard_normal((B, nin)).astype(np.float32)
+    U = rng.random((B, nu)).astype(np.float32)
+    h = L.MLP(nin, nh, nu, params=p0)
+    p, m, v = p0.astype(np.float64), np.zeros(len(p0)), np.zeros(len(p0))
+    large, none = np.ones(len(p0), bool), np.ones(len(p0), bool)
+    for t in range(1, steps + 1):
+        loss, g = h.grad(X, U)
+        g = g.astype(np.float64)
+        last = h.train(X, U, epochs=1, batch=B, lr=lr, seed=t)
+        assert abs(last - loss) <= 1e-5 * (1 + abs(loss))     # the loss is that of the batch before its step
+        m, v = 0.9 * m + 0.1 * g, 0.999 * v + 0.001 * g * g
+        p -= lr * (m / (1 - 0.9 ** t)) / (np.sqrt(v / (1 - 0.999 ** t)) + 1e-8)
+        large &= np.abs(g) >= 1e-3 * np.abs(g).max()
+        none &= g == 0
+    got = h.params()
+    d = np.abs(got - p)
+    assert large.mean() > 0.3
+    assert d[large].max() <= 0.02 * lr
+    assert d.max() <= 2 * lr * steps
+    np.testing.assert_array_equal(got[none], p0[none])
+    fresh = L.MLP(nin, nh, nu, params=got)
+    np.testing.assert_array_equal(h.forward(X[:B - 3]), fresh.forward(X[:B - 3]))
+    a, b = h.grad(X, U), fresh.grad(X, U)
+    assert a[0] == b[0]
+    np.testing.assert_array_equal(a[1], b[1])
+    h.close()
+    fresh.close()
+
+
 def test_mlp_training_reduces_loss():
     rng = np.random.default_rng(4)
     n, nin, nu = 8192, 64, 4
