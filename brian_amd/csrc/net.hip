@@ -74,6 +74,7 @@ struct HostGroup {
   DevBuf ptab_d;             // time-varying Poisson thresholds
   int64_t ptab_n0 = 0, ptab_len = 0;
   int ptab_per_neuron = 0;
+  double ptab_p = 0;         // mean spike probability of the table's entries
   std::vector<int> ssm_vars;         // variables recorded at spike times
   DevBuf ssm_d;
   DevBuf dlist_d, dcount_d, dbase_d, dsel_d;
@@ -192,6 +193,8 @@ struct bm_net {
   int route = 0;          // how the last run was launched (BM_TUNE_ROUTE)
   hipStream_t stream = nullptr;
   DevBuf d_base;          // int64 device step base
+  int small_req = 1;      // BM_TUNE_SMALL
+  bool small_on = false;  // runs take k_small (choose_small)
   JitKernel small;        // the whole network in one workgroup (net_small.hpp)
   DevBuf small_d;         // its descriptors, and what they were last copied from
   std::vector<unsigned char> small_h;
@@ -1001,7 +1004,8 @@ void run_persist(bm_net *net, int64_t nsteps) {
 // neurons FP64 4.6 -> 0.8, 4000 6.3 -> 2.0, 8000 6.9 -> 3.9, 8000 with 2000
 // synapses a neuron 15.6 -> 10.6; FP32 12,000 neurons 6.9 -> 3.0; 1000 Poisson
 // inputs with STDP onto 1 neuron 19.2 -> 1.3, onto 64 23.4 -> 2.0.  Beyond
-// 2^24 synapses one compute unit's reads of the rows would bound the step.
+// 2^24 synapses one compute unit's reads of the rows would bound the step even
+// where next to nothing spikes.
 int64_t small_neurons(const bm_net *net) { return net->precision == 32 ? 16384 : 8192; }
 constexpr int64_t SMALL_SYNAPSES = int64_t(1) << 24;
 // Runs of fewer steps keep the windowed kernels: one step takes 25 us either
@@ -1013,6 +1017,51 @@ int small_slots(const HostGroup &g) {      // neurons per thread, a power of two
   int k = 1;
   while ((int64_t)k * SMALL_THREADS < g.N) k *= 2;
   return k;
+}
+
+// Whether one workgroup is expected to advance the network faster than the
+// windows, whose workgroups share a step's deliveries out over the chip.  Times
+// of a step in us, fitted to networks of 500 to 12,000 neurons and 80 or 500
+// synapses a row at 300 to 30,000 (STDP: 100,000) deliveries a step:
+//   one workgroup  0.9 + 0.34 per 1000 neurons (FP32 0.95 + 0.23), and per 1000
+//                  deliveries 0.45, weights of their own 0.45 up to 4096 neurons,
+//                  0.8 beyond, in FP32 (no LDS instruction adds floats) 1.33; with
+//                  STDP 0.7, FP32 1.65
+//   windows        4.3, with STDP 14, and per 1000 deliveries 0.09 + 550 / sources,
+//                  with STDP 1.3 times that
+// Where the two meet, and the deliveries of the runs on either side (us a step,
+// one workgroup / windows): 2000 neurons 32,000 (30,000: 13.0 / 15.1); 4000 9200
+// (3000: 3.6 / 4.9, 30,000: 15.4 / 11.3); 8000 2300 (1000: 4.2 / 4.5, 10,000: 8.4 /
+// 5.8); FP32 weights of their own, 4000 neurons, 2700 (1000: 3.1 / 4.6, 10,000:
+// 14.9 / 6.9); 4000 inputs with STDP onto 4000 neurons 27,000 (10,000: 11.2 / 18.0,
+// 100,000: 68.6 / 51.0).
+// What a step delivers: Poisson sources at their rates (a table of rates at its
+// mean, where that is more); neurons, whose rates are not known beforehand, at
+// 100 Hz, which few networks reach.  At 300 Hz a network at the line takes up to
+// twice the windows' time in FP32 with weights of their own, 1.5 times else.
+constexpr double SMALL_RATE = 100.0;
+double spikes_per_step(const bm_net *net, const HostGroup &g, int64_t off, int64_t n) {
+  if (g.kind != GK_POISSON) return (double)n * std::min(1.0, SMALL_RATE * net->dt);
+  double s = 0;
+  for (int64_t i = off; i < off + n; ++i) s += (double)poisson_thr(g.rates[i] * net->dt) / 4294967296.0;
+  return g.ptab_len > 0 ? std::max(s, g.ptab_p * (double)n) : s;
+}
+bool small_pays(const bm_net *net) {
+  const bool f32 = net->precision == 32;
+  double N = 0;
+  for (auto &gp : net->groups) N += (double)gp->N;
+  double one = f32 ? 0.95 + 0.23e-3 * N : 0.9 + 0.34e-3 * N, win = net->stdps.empty() ? 4.3 : 14.0;
+  for (auto &cp : net->conns) {
+    const HostConn &c = *cp;
+    if (c.nnz == 0) continue;
+    const HostGroup &sg = *net->groups[c.src], &tg = *net->groups[c.tgt];
+    const bool stdp = c.stdp >= 0, count = tg.ring_desc[c.ring].kind == RING_COUNT;
+    double ev = spikes_per_step(net, sg, c.src_off, c.src_n) * (double)c.nnz / (double)c.src_n;
+    if (stdp) ev += spikes_per_step(net, tg, c.tgt_off, c.tgt_n) * (double)c.nnz / (double)c.tgt_n;
+    one += 1e-3 * ev * (stdp ? (f32 ? 1.65 : 0.7) : count || (!f32 && N <= 4096) ? 0.45 : f32 ? 1.33 : 0.8);
+    win += 1e-3 * ev * (0.09 + 550.0 / (double)sg.N) * (stdp ? 1.3 : 1.0);
+  }
+  return one <= win;
 }
 
 // LDS arrays of the network; returns the bytes in all.
@@ -1174,12 +1223,13 @@ std::string small_source(bm_net *net) {
   return d.str();
 }
 
-// Compiles (or takes from the cache) the one-workgroup kernel of an eligible
-// network.
-bool ensure_small(bm_net *net) {
-  if (!small_eligible(net)) return false;
-  if (!net->small.fn) net->small = jit_compile(small_source(net), "");
-  return true;
+// Decides whether the prepared network's runs take one workgroup, and compiles
+// (or takes from the cache) what they take: at prepare, and where rates or knobs
+// that the choice depends on change.
+void choose_small(bm_net *net) {
+  net->small_on = net->small_req != 0 && small_eligible(net) && (net->small_req == 2 || small_pays(net));
+  if (net->small_on && !net->small.fn) net->small = jit_compile(small_source(net), "");
+  if (!net->small_on) ensure_jit(net);
 }
 
 // One run in launches of at most SMALL_CHUNK steps; each applies the tail of
@@ -1885,7 +1935,7 @@ void prepare(bm_net *net, int window, int K, int use_graph) {
   check_launch_shapes(net);
   // a small network compiles its own kernel; its groups' sweeps, which only runs
   // of a few steps take, at the first such run
-  if (!ensure_small(net)) ensure_jit(net);
+  choose_small(net);
   net->d_base.alloc(8);
   int64_t zero = 0;
   BM_HIP(hipMemcpyAsync(net->d_base.p, &zero, 8, hipMemcpyHostToDevice, net->stream));
@@ -1923,7 +1973,7 @@ void run(bm_net *net, int64_t nsteps) {
     run_persist(net, nsteps);
     return;
   }
-  if (nsteps >= SMALL_MIN_STEPS && !net->profiling && ensure_small(net)) {
+  if (nsteps >= SMALL_MIN_STEPS && !net->profiling && net->small_on) {
     net->route = BM_ROUTE_ONE_WORKGROUP;
     run_small(net, nsteps);
     return;
@@ -2298,7 +2348,12 @@ int bm_net_set_poisson_rates(bm_net *net, int gid, int64_t first_step, int64_t n
     const int64_t width = per_neuron ? g.N : 1;
     BM_REQUIRE(nsteps * width <= (int64_t(1) << 28), "rate table too large");
     std::vector<uint64_t> thr((size_t)(nsteps * width));
-    for (size_t q = 0; q < thr.size(); ++q) thr[q] = poisson_thr(rates[q] * net->dt);
+    double p = 0;
+    for (size_t q = 0; q < thr.size(); ++q) {
+      thr[q] = poisson_thr(rates[q] * net->dt);
+      p += (double)thr[q] / 4294967296.0;
+    }
+    g.ptab_p = thr.empty() ? 0 : p / (double)thr.size();
     if (net->prepared) BM_HIP(hipStreamSynchronize(net->stream));   // launches in flight read the old table
     upload_raw(g.ptab_d, thr.data(), thr.size(), net->stream);
     g.ptab_n0 = first_step;
@@ -2313,6 +2368,7 @@ int bm_net_set_poisson_rates(bm_net *net, int gid, int64_t first_step, int64_t n
       net->graph_exec = nullptr;
       net->graph_windows = 0;
     }
+    if (net->prepared) choose_small(net);
   });
 }
 
@@ -2328,6 +2384,7 @@ int bm_net_set_poisson_base_rates(bm_net *net, int gid, const double *rates) {
     BM_REQUIRE(g.pthr_d.bytes == thr.size() * 8, "threshold buffer size");
     BM_HIP(hipMemcpyAsync(g.pthr_d.p, thr.data(), thr.size() * 8, hipMemcpyHostToDevice, net->stream));
     BM_HIP(hipStreamSynchronize(net->stream));
+    choose_small(net);
   });
 }
 
@@ -2860,6 +2917,7 @@ int bm_net_set_tuning(bm_net *net, int key, int value) {
         BM_REQUIRE(net->defer_W == 0 || value != 0, "deferred propagation needs the specialised kernels");
         BM_REQUIRE(!net->persist || value != 0, "persistent launches need the specialised kernels");
         net->specialize = value != 0;
+        if (net->prepared) choose_small(net);
         break;
       case BM_TUNE_DEFER:
         require_unprepared(net);
@@ -2868,6 +2926,13 @@ int bm_net_set_tuning(bm_net *net, int key, int value) {
       case BM_TUNE_LEAN:
         BM_REQUIRE(!net->persist || value != 0, "persistent launches need the lean kernels");
         net->lean_kernel = value != 0;
+        if (net->prepared) choose_small(net);
+        break;
+      case BM_TUNE_SMALL:
+        BM_REQUIRE(value >= 0 && value <= 2, "small must be 0 (never), 1 (where it is expected to be faster) or 2 (wherever "
+                                             "the network fits)");
+        net->small_req = value;
+        if (net->prepared) choose_small(net);
         break;
       case BM_TUNE_PERSIST:
         if (value != 0) {
@@ -2926,6 +2991,7 @@ int bm_net_get_tuning(bm_net *net, int key, int *value) {
       case BM_TUNE_PERSIST_CHUNK: *value = net->persist_chunk; break;
       case BM_TUNE_PERSIST_QUEUE: *value = net->persist_queue; break;
       case BM_TUNE_ROUTE: *value = net->route; break;
+      case BM_TUNE_SMALL: *value = net->small_req; break;
       default: throw Error(BM_EINVAL, "unknown tuning key");
     }
   });

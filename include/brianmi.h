@@ -323,10 +323,7 @@ int bm_net_set_partition(bm_net *net, int gid, int nparts, const int64_t *offset
  *                              ring layout, channel table, resets and threshold
  *                              as constants, a nonlinear model's program as code;
  *                              0: the precompiled generic form, programs
- *                              interpreted.  With it (and BM_TUNE_LEAN) runs of 4
- *                              steps or more of a small network that takes a
- *                              launch per step (a connection without delay, or
- *                              STDP) are one launch of one workgroup
+ *                              interpreted
  *   BM_TUNE_DEFER              (before prepare) 1: specialised lean groups
  *                              deliver each window's spikes during the next
  *                              launch, half of the workgroups before and half
@@ -360,6 +357,14 @@ int bm_net_set_partition(bm_net *net, int gid, int nparts, const int64_t *offset
  *                              ring instead, so results never depend on it;
  *                              the queues take D x N x value / 16 x 4 bytes,
  *                              allocated at the first persistent run
+ *   BM_TUNE_SMALL              with BM_TUNE_SPECIALIZE and BM_TUNE_LEAN, runs of 4
+ *                              steps or more of a small network that otherwise
+ *                              takes a launch per step (a connection without
+ *                              delay, or STDP) are one launch of one workgroup:
+ *                              1 (default) where that is expected to be faster
+ *                              with its neurons spiking at up to 100 Hz and its
+ *                              Poisson sources at their rates, 2 wherever the
+ *                              network fits, 0 never
  *   BM_TUNE_ROUTE              (get only) how the last run was launched: 0 no run
  *                              yet, BM_ROUTE_WINDOWS (a launch per group and
  *                              window), BM_ROUTE_ONE_WORKGROUP (the whole network
@@ -380,7 +385,8 @@ enum {
   BM_TUNE_PERSIST = 12,
   BM_TUNE_PERSIST_CHUNK = 13,
   BM_TUNE_PERSIST_QUEUE = 14,
-  BM_TUNE_ROUTE = 15
+  BM_TUNE_ROUTE = 15,
+  BM_TUNE_SMALL = 16
 };
 enum { BM_ROUTE_WINDOWS = 1, BM_ROUTE_ONE_WORKGROUP = 2 };
 int bm_net_set_tuning(bm_net *net, int key, int value);

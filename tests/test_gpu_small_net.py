@@ -1,9 +1,8 @@
-"""Small networks in one workgroup (net_small.hpp) against the windowed
-kernels, which runs of fewer than 4 steps take: the same network run in long
-stretches, and in stretches of at most 3 steps.  Deliveries that are counts:
-rasters and state equal bit for bit; weights per synapse: equal up to the order
-of the floating additions (a handful of values per target and step, so 1e-12
-relative in FP64)."""
+"""Small networks in one workgroup (net_small.hpp; BM_TUNE_SMALL 2) against
+the windowed kernels (BM_TUNE_SMALL 0), each arm's route checked.  Deliveries
+that are counts: rasters and state equal bit for bit; weights per synapse: equal
+up to the order of the floating additions (a handful of values per target and
+step, so 1e-12 relative in FP64).  Then where the one or the other is taken."""
 import numpy as np
 import pytest
 
@@ -22,21 +21,21 @@ def _csr(rng, nsrc, ntgt, p):
     return ptr, np.nonzero(m)[1]
 
 
-def _advance(h, stretches, small):
+WINDOWS, ONE_WORKGROUP = 1, 2
+
+
+def _advance(h, stretches, small, fits=True):
+    h.set_tuning("small", 2 if small else 0)
     for s in stretches:
-        if small:
-            h.run(s)
-        else:
-            while s > 0:
-                h.run(min(s, 3))
-                s -= min(s, 3)
+        h.run(s)
+        assert h.get_tuning("route") == (ONE_WORKGROUP if small and fits and s >= 4 else WINDOWS)
 
 
-def _both(build, stretches, exact=True, rtol=1e-12):
+def _both(build, stretches, exact=True, rtol=1e-12, fits=True):
     out = []
     for small in (True, False):
         h, read = build()
-        _advance(h, stretches, small)
+        _advance(h, stretches, small, fits)
         out.append(read(h))
         h.close()
     assert len(out[0]) == len(out[1])
@@ -91,7 +90,8 @@ def test_count_network(n, kind, precision):
         h.prepare()
         return h, lambda h: [*h.get_spikes(g), *[h.get_state(g, v, n) for v in range(4)]]
 
-    out = _both(build, (2, 300, 1, 4, 250))
+    # 8192 neurons in FP64 and 16,384 in FP32, as far as the rings fit the LDS
+    out = _both(build, (2, 300, 1, 4, 250), fits=precision == 32 or n <= 8192)
     if n > 1:
         assert len(out[0]) > 5
 
@@ -218,3 +218,80 @@ def test_raster_regions_fill_evenly():
 
     out = _both(build, [32] * runs)
     assert len(out[0]) > n * 32 * runs // 160
+
+
+def _deliveries(n, row, precision=64, exact_weights=True, poisson=None, stdp=False):
+    """n neurons (or Poisson sources at a rate, and n neurons) with `row`
+    synapses each and no delay."""
+    rng = np.random.default_rng(n + row)
+    h = NetHandle(DT, precision)
+    src = None if poisson is None else h.add_poisson(n, np.full(n, float(poisson)), 5)
+    S0 = np.zeros((2, n))
+    S0[0] = rng.random(n)
+    g = h.add_group(S0)
+    h.set_linear(g, np.diag([1.0, 0.9]), np.array([0.01 if poisson is None else 0.0, 0.0]))
+    h.set_threshold(g, 0, 1.0)
+    h.add_reset_op(g, 0, 0, 0.0)
+    col = np.sort(rng.integers(0, n, (n, row)), axis=1).ravel()
+    w = np.full(n * row, 1e-3) if exact_weights else 1e-3 * rng.random(n * row)
+    c = h.add_connection(g if src is None else src, 0, n, g, 0, n, 1, np.arange(n + 1) * row, col, w)
+    if stdp:
+        h.add_stdp(c, 0.99, 0.99, 1e-5, -1e-5, 0.0, 1e-3, 0, 0)
+    h.record(g, n * 64)
+    h.prepare()
+    return h, src, g
+
+
+@pytest.mark.parametrize("n,row,precision,exact_weights,stdp,route", [
+    # at 100 Hz: 10,000 deliveries a step of 1000 neurons, 3200 and 20,000 of 4000,
+    # 6400 of 8000
+    (1000, 1000, 64, True, False, ONE_WORKGROUP), (4000, 80, 64, True, False, ONE_WORKGROUP),
+    (4000, 500, 64, True, False, WINDOWS), (8000, 80, 64, True, False, WINDOWS),
+    (8000, 20, 64, True, False, ONE_WORKGROUP), (8000, 2000, 64, True, False, WINDOWS),
+    (2000, 100, 32, False, False, ONE_WORKGROUP), (4000, 80, 32, False, False, WINDOWS),
+    (4000, 80, 64, False, False, ONE_WORKGROUP)])
+def test_dense_networks_keep_the_windows(n, row, precision, exact_weights, stdp, route):
+    h, _, g = _deliveries(n, row, precision, exact_weights, stdp=stdp)
+    assert h.get_tuning("small") == 1
+    h.run(8)
+    assert h.get_tuning("route") == route
+    a = h.get_spikes(g)
+    h.close()
+    h, _, g = _deliveries(n, row, precision, exact_weights, stdp=stdp)
+    h.set_tuning("small", 2 if route == WINDOWS else 0)
+    h.run(8)
+    assert h.get_tuning("route") == (ONE_WORKGROUP if route == WINDOWS else WINDOWS)
+    for x, y in zip(a, h.get_spikes(g)):        # the potentials do not see the deliveries
+        np.testing.assert_array_equal(x, y)
+    h.close()
+
+
+@pytest.mark.parametrize("stdp", [False, True])
+def test_poisson_rates_choose_the_kernel(stdp):
+    """Sources at 20 Hz leave a step little to deliver, at 4000 Hz much; base
+    rates and tables set between runs count, and switching changes nothing but
+    the kernel."""
+    out = []
+    for small in (1, 0):
+        h, p, g = _deliveries(2000, 500 if stdp else 100, 64, False, poisson=20, stdp=stdp)
+        h.set_tuning("small", small)
+        routes = []
+        for rates, table in ((None, None), (4000.0, None), (20.0, None), (None, 4000.0)):
+            if rates is not None:
+                h.set_poisson_base_rates(p, np.full(2000, rates))
+            if table is not None:
+                h.set_poisson_rates(p, 0, np.full(40, table), False)
+            h.run(8)
+            routes.append(h.get_tuning("route"))
+        assert routes == ([ONE_WORKGROUP, WINDOWS, ONE_WORKGROUP, WINDOWS] if small else [WINDOWS] * 4)
+        out.append(h.get_state(g, 1, 2000))
+        h.close()
+    np.testing.assert_allclose(out[0], out[1], rtol=1e-12)
+
+
+def test_small_refuses_other_values():
+    h, _, _ = _deliveries(100, 5)
+    for v in (-1, 3):
+        with pytest.raises(Exception, match="small must be"):
+            h.set_tuning("small", v)
+    h.close()
