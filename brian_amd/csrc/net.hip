@@ -194,7 +194,8 @@ struct bm_net {
   hipStream_t stream = nullptr;
   DevBuf d_base;          // int64 device step base
   int small_req = 1;      // BM_TUNE_SMALL
-  bool small_on = false;  // runs take k_small (choose_small)
+  bool small_on = false;  // runs of at least small_min steps take k_small (choose_small)
+  int64_t small_min = 0;
   JitKernel small;        // the whole network in one workgroup (net_small.hpp)
   DevBuf small_d;         // its descriptors, and what they were last copied from
   std::vector<unsigned char> small_h;
@@ -1001,17 +1002,25 @@ void run_persist(bm_net *net, int64_t nsteps) {
 // and 16 in FP32 keep the state of 3 variables within the 128 registers of a
 // 1024-thread workgroup (and the rings must fit its LDS: about 15,000 neurons
 // without delays).  us a step, windowed -> here, CUBA network without delays: 1000
-// neurons FP64 4.6 -> 0.8, 4000 6.3 -> 2.0, 8000 6.9 -> 3.9, 8000 with 2000
-// synapses a neuron 15.6 -> 10.6; FP32 12,000 neurons 6.9 -> 3.0; 1000 Poisson
-// inputs with STDP onto 1 neuron 19.2 -> 1.3, onto 64 23.4 -> 2.0.  Beyond
+// neurons FP64 4.6 -> 0.8, 4000 6.3 -> 2.0, 8000 6.9 -> 3.9; FP32 12,000 neurons
+// 6.9 -> 3.0; 1000 Poisson inputs with STDP onto 1 neuron 19.2 -> 1.3, onto 64 23.4 -> 2.0.  Beyond
 // 2^24 synapses one compute unit's reads of the rows would bound the step even
 // where next to nothing spikes.
 int64_t small_neurons(const bm_net *net) { return net->precision == 32 ? 16384 : 8192; }
 constexpr int64_t SMALL_SYNAPSES = int64_t(1) << 24;
-// Runs of fewer steps keep the windowed kernels: one step takes 25 us either
-// way (launches there, loading and storing the network's state and rings here);
-// 4 steps of 12,000 neurons 50 us windowed, of 4000 neurons 72.
-constexpr int64_t SMALL_MIN_STEPS = 4;
+// Networks of more neurons than this keep the windows for runs of fewer than 4
+// steps: loading and storing the network's state and rings costs a launch of one
+// workgroup more than the windows' launches do (us of a run of 1 and of 3 steps
+// and its synchronization, one workgroup / windows: 8000 neurons FP64 27 / 21 and
+// 32 / 31, 12,000 FP32 28 / 21 and 33 / 31; 4000 FP64 21 / 22 and 24 / 32, 1000 15
+// / 20 and 17 / 27).  They compile both kernels when they are prepared; smaller
+// ones need no other.
+constexpr int64_t SMALL_SHORT_NEURONS = 4096;
+int64_t small_min_steps(const bm_net *net) {
+  int64_t N = 0;
+  for (auto &gp : net->groups) N += gp->N;
+  return N <= SMALL_SHORT_NEURONS ? 1 : 4;
+}
 
 int small_slots(const HostGroup &g) {      // neurons per thread, a power of two
   int k = 1;
@@ -1229,7 +1238,8 @@ std::string small_source(bm_net *net) {
 void choose_small(bm_net *net) {
   net->small_on = net->small_req != 0 && small_eligible(net) && (net->small_req == 2 || small_pays(net));
   if (net->small_on && !net->small.fn) net->small = jit_compile(small_source(net), "");
-  if (!net->small_on) ensure_jit(net);
+  net->small_min = net->small_on ? small_min_steps(net) : 0;
+  if (net->small_min != 1) ensure_jit(net);
 }
 
 // One run in launches of at most SMALL_CHUNK steps; each applies the tail of
@@ -1933,8 +1943,6 @@ void prepare(bm_net *net, int window, int K, int use_graph) {
     net->lates.push_back(lm);
   }
   check_launch_shapes(net);
-  // a small network compiles its own kernel; its groups' sweeps, which only runs
-  // of a few steps take, at the first such run
   choose_small(net);
   net->d_base.alloc(8);
   int64_t zero = 0;
@@ -1973,7 +1981,7 @@ void run(bm_net *net, int64_t nsteps) {
     run_persist(net, nsteps);
     return;
   }
-  if (nsteps >= SMALL_MIN_STEPS && !net->profiling && net->small_on) {
+  if (net->small_on && nsteps >= net->small_min && !net->profiling) {
     net->route = BM_ROUTE_ONE_WORKGROUP;
     run_small(net, nsteps);
     return;
@@ -3243,6 +3251,7 @@ int bm_net_get_stdp_traces(bm_net *net, int sid, double *a_pre, double *a_post) 
 int bm_net_set_profiling(bm_net *net, int enable) {
   return guard([&] {
     net->profiling = enable != 0;
+    if (net->prepared && net->profiling) ensure_jit(net);   // profiled runs take the windows
     net->prof_launches = 0;
     net->prof_ms = 0;
   });

@@ -357,10 +357,11 @@ int bm_net_set_partition(bm_net *net, int gid, int nparts, const int64_t *offset
  *                              ring instead, so results never depend on it;
  *                              the queues take D x N x value / 16 x 4 bytes,
  *                              allocated at the first persistent run
- *   BM_TUNE_SMALL              with BM_TUNE_SPECIALIZE and BM_TUNE_LEAN, runs of 4
- *                              steps or more of a small network that otherwise
- *                              takes a launch per step (a connection without
- *                              delay, or STDP) are one launch of one workgroup:
+ *   BM_TUNE_SMALL              with BM_TUNE_SPECIALIZE and BM_TUNE_LEAN, a run of a
+ *                              small network that otherwise takes a launch per
+ *                              step (a connection without delay, or STDP) is one
+ *                              launch of one workgroup (above 4096 neurons only
+ *                              a run of at least 4 steps):
  *                              1 (default) where that is expected to be faster
  *                              with its neurons spiking at up to 100 Hz and its
  *                              Poisson sources at their rates, 2 wherever the

@@ -3,6 +3,8 @@ the windowed kernels (BM_TUNE_SMALL 0), each arm's route checked.  Deliveries
 that are counts: rasters and state equal bit for bit; weights per synapse: equal
 up to the order of the floating additions (a handful of values per target and
 step, so 1e-12 relative in FP64).  Then where the one or the other is taken."""
+import time
+
 import numpy as np
 import pytest
 
@@ -24,18 +26,18 @@ def _csr(rng, nsrc, ntgt, p):
 WINDOWS, ONE_WORKGROUP = 1, 2
 
 
-def _advance(h, stretches, small, fits=True):
+def _advance(h, stretches, small, fits=True, shortest=1):
     h.set_tuning("small", 2 if small else 0)
     for s in stretches:
         h.run(s)
-        assert h.get_tuning("route") == (ONE_WORKGROUP if small and fits and s >= 4 else WINDOWS)
+        assert h.get_tuning("route") == (ONE_WORKGROUP if small and fits and s >= shortest else WINDOWS)
 
 
-def _both(build, stretches, exact=True, rtol=1e-12, fits=True):
+def _both(build, stretches, exact=True, rtol=1e-12, fits=True, shortest=1):
     out = []
     for small in (True, False):
         h, read = build()
-        _advance(h, stretches, small, fits)
+        _advance(h, stretches, small, fits, shortest)
         out.append(read(h))
         h.close()
     assert len(out[0]) == len(out[1])
@@ -91,7 +93,7 @@ def test_count_network(n, kind, precision):
         return h, lambda h: [*h.get_spikes(g), *[h.get_state(g, v, n) for v in range(4)]]
 
     # 8192 neurons in FP64 and 16,384 in FP32, as far as the rings fit the LDS
-    out = _both(build, (2, 300, 1, 4, 250), fits=precision == 32 or n <= 8192)
+    out = _both(build, (2, 300, 1, 4, 250), fits=precision == 32 or n <= 8192, shortest=1 if n <= 4096 else 4)
     if n > 1:
         assert len(out[0]) > 5
 
@@ -167,9 +169,9 @@ def test_long_run_and_rate_changes():
 
 
 @pytest.mark.parametrize("vt", [np.inf, -np.inf, np.nan])
-@pytest.mark.parametrize("steps", [3, 40])     # windowed kernels, one workgroup
+@pytest.mark.parametrize("small", [0, 2])      # windowed kernels, one workgroup
 @pytest.mark.parametrize("kind", ["counts", "weights", "program"])
-def test_constants_without_a_literal(kind, steps, vt):
+def test_constants_without_a_literal(kind, small, vt):
     """Thresholds and reset values that are infinite or NaN, against the kernels
     that read them from tables (specialize 0)."""
     out = []
@@ -191,8 +193,10 @@ def test_constants_without_a_literal(kind, steps, vt):
         h.add_connection(g, 0, n, g, 0, n, 0, np.arange(n + 1), np.arange(n), w)
         h.record(g, 1 << 14)
         h.prepare()
+        h.set_tuning("small", small)
         h.set_tuning("specialize", specialize)
-        h.run(steps)
+        h.run(40)
+        assert h.get_tuning("route") == (ONE_WORKGROUP if small and specialize and kind != "program" else WINDOWS)
         out.append([*h.get_spikes(g), h.get_state(g, 0, n), h.get_state(g, 1, n)])
         h.close()
     assert len(out[0][0]) == (0 if kind != "program" and not vt < 0 else len(out[1][0]))
@@ -263,6 +267,29 @@ def test_dense_networks_keep_the_windows(n, row, precision, exact_weights, stdp,
     assert h.get_tuning("route") == (ONE_WORKGROUP if route == WINDOWS else WINDOWS)
     for x, y in zip(a, h.get_spikes(g)):        # the potentials do not see the deliveries
         np.testing.assert_array_equal(x, y)
+    h.close()
+
+
+@pytest.mark.parametrize("n", [4096, 4097])
+def test_first_short_run_compiles_nothing(n):
+    """Runs of 1 to 3 steps, as of scripts that go on step by step, find their
+    kernel compiled at prepare: 0.1 s and more for a network whose constants no
+    cache knows, where a step takes under 0.1 ms."""
+    A = 0.9 + 0.05 * np.random.default_rng().random()
+    h = NetHandle(DT, 64)
+    g = h.add_group(np.random.default_rng(0).random((1, n)))
+    h.set_linear(g, np.array([[A]]), np.array([0.2]))
+    h.set_threshold(g, 0, 1.0)
+    h.add_reset_op(g, 0, 0, 0.0)
+    h.add_connection(g, 0, 1, g, 0, n, 0, np.array([0, 1]), np.array([0]), np.array([1e-3]))
+    h.prepare()
+    h.sync()
+    for steps in (1, 3, 8, 2):
+        t = time.perf_counter()
+        h.run(steps)
+        h.sync()
+        assert time.perf_counter() - t < 0.03
+        assert h.get_tuning("route") == (WINDOWS if n > 4096 and steps < 4 else ONE_WORKGROUP)
     h.close()
 
 
