@@ -27,7 +27,7 @@ Pi64 = C.POINTER(C.c_int64)
 TUNE = {"window": 1, "neurons_per_thread": 2, "wave_max": 3, "row_split": 4, "ring_bits": 5,
         "ring_pack": 6, "use_graph": 7, "window_max": 8, "specialize": 9, "defer": 10, "lean": 11,
         "persist": 12, "persist_chunk": 13, "persist_queue": 14, "route": 15,
-        "small": 16}
+        "small": 16, "compiled": 17}
 
 
 class BrianMIError(RuntimeError):

@@ -53,4 +53,17 @@ __host__ __device__ inline uint32_t weyl_u32(uint32_t key, uint32_t counter) {
   return h;
 }
 
+#if defined(__HIPCC__) || defined(__HIPCC_RTC__)
+// a value that is the same in all lanes, in a scalar register
+__device__ __forceinline__ float uniform(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double uniform(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+#endif
+
 }  // namespace bm

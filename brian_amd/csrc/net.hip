@@ -25,8 +25,17 @@ static thread_local std::string g_last_error;
 void set_last_error(const std::string &msg) { g_last_error = msg; }
 
 // a module compiled at run time and the kernel in it
-struct JitKernel {
+struct JitModule {
   hipModule_t mod = nullptr;
+  int64_t used = 0;       // when a handle last took it (JitCache)
+  JitModule() = default;
+  JitModule(const JitModule &) = delete;
+  ~JitModule() {
+    if (mod) (void)hipModuleUnload(mod);
+  }
+};
+struct JitKernel {
+  std::shared_ptr<JitModule> mod;
   hipFunction_t fn = nullptr;
 };
 
@@ -453,9 +462,33 @@ void check_launch_shapes(bm_net *net) {
 // ---- lean sweep specialised at run time (hipRTC)
 // The lean kernel's ring layout, channel table, reset ops and threshold are
 // fixed per group; compiled with those as constants the kernel carries no
-// per-step table lookups.  Modules are cached per source for the process.
-std::mutex g_jit_mu;
-std::map<std::string, JitKernel> g_jit;
+// per-step table lookups.  Modules are cached per source for the process: those
+// that handles hold, and the JIT_IDLE last used of the others.
+constexpr size_t JIT_IDLE = 32;
+struct JitCache {
+  std::mutex mu;
+  std::map<std::string, JitKernel> kernels;
+  int64_t clock = 0, compiled = 0;
+};
+JitCache &jit_cache() {
+  static JitCache *c = new JitCache;    // not destroyed: the HIP runtime may be gone by then
+  return *c;
+}
+// Unloads the longest unused modules that no handle holds, beyond JIT_IDLE of
+// them.  A handle drops a module it has launched when a knob changes its kernels,
+// so the launches in flight are waited for first.
+void jit_trim(JitCache &c) {
+  std::vector<std::pair<int64_t, const std::string *>> idle;
+  for (const auto &e : c.kernels)
+    if (e.second.mod.use_count() == 1) idle.push_back({e.second.mod->used, &e.first});
+  if (idle.size() <= JIT_IDLE) return;
+  if (hipDeviceSynchronize() != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  std::sort(idle.begin(), idle.end());
+  for (size_t q = 0; q + JIT_IDLE < idle.size(); ++q) c.kernels.erase(c.kernels.find(*idle[q].second));
+}
 
 std::string jit_list(const std::vector<int> &v) {
   std::ostringstream o;
@@ -529,6 +562,54 @@ std::string prog_prelude(bm_net *net, const HostGroup &g) {
   return d.str();
 }
 
+// How a group's constants enter its code: written out as literals, or read once
+// a launch from the group's descriptor into a struct (`kv`), so that networks
+// that differ in nothing else share one compiled kernel.  A program that builds
+// its network anew for each value of a parameter compiles the latter once (0.17 s
+// a kernel, which 1000 Poisson inputs with STDP repay in some 10,000 steps).
+// Literals are for the common shape, where they shorten the step (4000 neurons,
+// FP64, one workgroup: 2.89 us a step with literals, 2.97 without), and for
+// nonlinear programs, whose constants fold (compiling repays within 400 steps).
+struct Consts {
+  const HostGroup &g;
+  bool f32, table;
+  std::string of(double v, const char *field, size_t q) const {
+    return table ? std::string("kv.") + field + "[" + std::to_string(q) + "]" : lit(v, f32);
+  }
+  std::string A(size_t q) const { return of(g.A[q], "A", q); }
+  std::string C(size_t q) const { return of(g.C[q], "C", q); }
+  std::string vt() const { return of(g.vt, "vt", 0); }
+  std::string rs(size_t q) const { return of(g.rs_val[q], "rs", q); }
+  std::string w(size_t q) const { return of(g.chans[q].w, "w", q); }
+};
+
+Consts consts(const bm_net *net, const HostGroup &g) {
+  return {g, net->precision == 32, !lean_shape(g) && g.upd != UPD_PROGRAM};
+}
+
+void emit_values(std::ostringstream &d, const Consts &k, const std::string &name, const std::string &type) {
+  d << "struct " << name << " {\n";
+  const std::pair<const char *, size_t> fields[] = {
+      {"A", k.g.A.size()}, {"C", k.g.C.size()}, {"rs", k.g.rs_val.size()}, {"w", k.g.chans.size()}};
+  if (k.table) {
+    for (const auto &f : fields) d << "  " << type << " " << f.first << "[" << std::max<size_t>(f.second, 1) << "];\n";
+    d << "  " << type << " vt[1];\n";
+  }
+  d << "  __device__ __forceinline__ explicit " << name << "(const GroupDev &g) {\n";
+  if (k.table) {
+    for (const auto &f : fields)
+      for (size_t q = 0; q < f.second; ++q) {
+        const std::string at = "[" + std::to_string(q) + "]";
+        const std::string from = f.first == std::string("rs") ? "g.rs_val" + at
+                                 : f.first == std::string("w") ? "g.chans" + at + ".w"
+                                                               : std::string("g.") + f.first + at;
+        d << "    " << f.first << at << " = uniform((" << type << ")" << from << ");\n";
+      }
+    d << "    vt[0] = uniform((" << type << ")g.vt);\n";
+  }
+  d << "  }\n};\n";
+}
+
 // The pieces of a group's model as code.
 // Deliveries in the channel order (Connections, then DelayConnection
 // flushes), from one packed count word.
@@ -551,12 +632,12 @@ void emit_deliver(std::ostringstream &d, bm_net *net, const HostGroup &g) {
 // values f of each, in the channel order.  Groups with one count ring keep
 // k_lean's arithmetic (FP32: one fused multiply-add per channel), the others
 // the general sweep's, which they otherwise run.
-void emit_deliver_rings(std::ostringstream &d, bm_net *net, const HostGroup &g, const std::string &head,
-                        const std::string &type) {
-  const bool f32 = net->precision == 32;
+void emit_deliver_rings(std::ostringstream &d, const Consts &k, const std::string &head, const std::string &type) {
+  const HostGroup &g = k.g;
   d << head << " {\n";
   if (g.kind == GK_NEURON)
-    for (const ChanDev &c : g.chans) {
+    for (size_t q = 0; q < g.chans.size(); ++q) {
+      const ChanDev &c = g.chans[q];
       const RingDev &rd = g.ring_desc[c.ring];
       const std::string x = "x[" + std::to_string(c.var) + "]";
       if (rd.kind != RING_COUNT) {
@@ -566,55 +647,55 @@ void emit_deliver_rings(std::ostringstream &d, bm_net *net, const HostGroup &g, 
       const uint32_t mask = rd.bits >= 32 ? 0xFFFFFFFFu : ((1u << rd.bits) - 1u);
       const std::string cnt =
           "((w[" + std::to_string(c.ring) + "] >> " + std::to_string(c.ch * rd.bits) + ") & " + std::to_string(mask) + "u)";
-      if (f32 && one_count_ring(g)) d << "    " << x << " = __builtin_fmaf((float)" << cnt << ", " << lit(c.w, true) << ", " << x << ");\n";
-      else d << "    " << x << " = apply_count<" << type << ">(" << x << ", " << cnt << ", " << lit(c.w, f32) << ", " << c.is_delay << ");\n";
+      if (k.f32 && one_count_ring(g)) d << "    " << x << " = __builtin_fmaf((float)" << cnt << ", " << k.w(q) << ", " << x << ");\n";
+      else d << "    " << x << " = apply_count<" << type << ">(" << x << ", " << cnt << ", " << k.w(q) << ", " << c.is_delay << ");\n";
     }
   d << "  }\n";
 }
 
-void emit_reset(std::ostringstream &d, bm_net *net, const HostGroup &g, const std::string &head) {
+void emit_reset(std::ostringstream &d, const Consts &k, const std::string &head) {
+  const HostGroup &g = k.g;
   d << head << " {\n";
   for (size_t r = 0; r < g.rs_var.size(); ++r) {
-    const std::string v =
-        g.rs_vvar[r] >= 0 ? "x[" + std::to_string(g.rs_vvar[r]) + "]" : lit(g.rs_val[r], net->precision == 32);
+    const std::string v = g.rs_vvar[r] >= 0 ? "x[" + std::to_string(g.rs_vvar[r]) + "]" : k.rs(r);
     if (g.rs_op[r] == 0) d << "  x[" << g.rs_var[r] << "] = " << v << ";\n";
     else d << "  x[" << g.rs_var[r] << "] = x[" << g.rs_var[r] << "] + " << v << ";\n";
   }
   d << "}\n";
 }
 
-void emit_linear(std::ostringstream &d, bm_net *net, const HostGroup &g, const std::string &head,
-                 const std::string &type) {
+void emit_linear(std::ostringstream &d, const Consts &k, const std::string &head, const std::string &type) {
+  const HostGroup &g = k.g;
   const int M = g.M;
   d << head << " {\n";
-  if (net->precision == 32 && !one_count_ring(g)) {
+  if (k.f32 && !one_count_ring(g)) {
     // the general sweep's order, which such groups otherwise run
     d << "  const " << type << " a[" << M * M << "] = {";
-    for (int q = 0; q < M * M; ++q) d << (q ? "," : "") << lit(g.A[q], true);
+    for (int q = 0; q < M * M; ++q) d << (q ? "," : "") << k.A(q);
     d << "}, c[" << M << "] = {";
-    for (int q = 0; q < M; ++q) d << (q ? "," : "") << lit(g.C[q], true);
+    for (int q = 0; q < M; ++q) d << (q ? "," : "") << k.C(q);
     d << "};\n  " << type << " s[" << M << "][1];\n  for (int j = 0; j < " << M << "; ++j) s[j][0] = x[j];\n  linear_exact<" << M
       << ", 1>(s, a, c);\n  for (int j = 0; j < " << M << "; ++j) x[j] = s[j][0];\n";
-  } else if (net->precision == 64) {
+  } else if (!k.f32) {
     // S <- A.S + C as the left fold A[j,0]*S0 + A[j,1]*S1 + ..., then + C[j]
     // (brian/stateupdater.py:413-416 in that order), no contraction
     d << "#pragma clang fp contract(off)\n";
     for (int j = 0; j < M; ++j) {
       d << "  const " << type << " t" << j << " = ";
-      for (int q = 0; q < M; ++q) d << (q ? " + " : "") << lit(g.A[j * M + q], false) << " * x[" << q << "]";
+      for (int q = 0; q < M; ++q) d << (q ? " + " : "") << k.A(j * M + q) << " * x[" << q << "]";
       d << ";\n";
     }
-    for (int j = 0; j < M; ++j) d << "  x[" << j << "] = t" << j << " + " << lit(g.C[j], false) << ";\n";
+    for (int j = 0; j < M; ++j) d << "  x[" << j << "] = t" << j << " + " << k.C(j) << ";\n";
   } else {
     for (int j = 0; j < M; ++j) {
       std::string e;
-      if (g.C[j] != 0.0) e = lit(g.C[j], true);
+      if (g.C[j] != 0.0) e = k.C(j);
       for (int q = 0; q < M; ++q) {
         const double a = g.A[j * M + q];
         if (a == 0.0) continue;
         const std::string term = "x[" + std::to_string(q) + "]";
-        if (e.empty()) e = (a == 1.0) ? term : lit(a, true) + " * " + term;
-        else e = "__builtin_fmaf(" + lit(a, true) + ", " + term + ", " + e + ")";
+        if (e.empty()) e = (a == 1.0) ? term : k.A(j * M + q) + " * " + term;
+        else e = "__builtin_fmaf(" + k.A(j * M + q) + ", " + term + ", " + e + ")";
       }
       d << "  const " << type << " t" << j << " = " << (e.empty() ? "0.0f" : e) << ";\n";
     }
@@ -623,17 +704,17 @@ void emit_linear(std::ostringstream &d, bm_net *net, const HostGroup &g, const s
   d << "}\n";
 }
 
-void emit_spike(std::ostringstream &d, bm_net *net, const HostGroup &g, const std::string &head) {
+void emit_spike(std::ostringstream &d, const Consts &k, const std::string &head) {
+  const HostGroup &g = k.g;
   d << head << " { return ";
   if (g.th_kind == TH_NONE) d << "false";   // a group without a threshold never spikes
   else if (g.th_kind == TH_VAR) d << "x[" << g.th_var << "] > x[" << g.th_vtvar << "]";
-  else d << "x[" << g.th_var << "] > " << lit(g.vt, net->precision == 32);
+  else d << "x[" << g.th_var << "] > " << k.vt();
   d << "; }\n";
 }
 
 // The group's model as compile-time code for k_lean (net_lean.hpp): the
-// channel deliveries, reset ops, linear update and threshold of this group
-// with every constant written out.  FP64 keeps the reference's arithmetic
+// channel deliveries, reset ops, linear update and threshold of this group.  FP64 keeps the reference's arithmetic
 // (count loops, left-fold rows with no contraction); FP32 uses one fused
 // multiply-add per delivery and per non-zero entry of A.
 std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_header = "net_lean.hpp") {
@@ -652,26 +733,28 @@ std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_hea
     << "typedef " << (f32 ? "float" : "double") << " lean_t;\n#define LEAN_WMAX " << net->Wcap
     << "\n#define LEAN_NRING " << nring << "\n#define LEAN_POISSON " << (g.kind == GK_POISSON ? 1 : 0)
     << "\nconstexpr int lean_count[] = {" << each([](const RingDev &r) { return r.kind == RING_COUNT ? 1 : 0; })
-    << "}, lean_sw[] = {" << each([](const RingDev &r) { return r.sw; }) << "};\n#define LEAN_EMP " << (g.th_kind == TH_EMPIRICAL ? g.th_period : -1) << "\n#define LEAN_M " << M << "\n#define LEAN_SW " << sw
+    << "}, lean_sw[] = {" << each([](const RingDev &r) { return r.sw; }) << "};\n#define LEAN_EMP " << (g.th_kind == TH_EMPIRICAL ? 1 : 0) << "\n#define LEAN_M " << M << "\n#define LEAN_SW " << sw
     << "\n#define LEAN_REFR " << (g.refr == REFR_CONST ? 1 : (g.refr == REFR_ARRAY ? 2 : 0)) << "\n";
+  const Consts k = consts(net, g);
+  emit_values(d, k, "lean_kv", "lean_t");
   if (g.kind == GK_POISSON) {
     d << "}\n#include \"" << kernel_header << "\"\n";
     return d.str();
   }
-  emit_deliver(d, net, g);
-  emit_deliver_rings(d, net, g, "__device__ inline void lean_deliver_rings(lean_t (&x)[LEAN_M], const uint32_t (&w)[" +
-                     std::to_string(std::max(nring, 1)) + "], const lean_t (&f)[" + std::to_string(std::max(nring, 1)) + "])",
+  if (kernel_header != std::string("net_lean.hpp")) emit_deliver(d, net, g);   // k_persist: one packed count word
+  emit_deliver_rings(d, k, "__device__ inline void lean_deliver_rings(lean_t (&x)[LEAN_M], const uint32_t (&w)[" +
+                     std::to_string(std::max(nring, 1)) + "], const lean_t (&f)[" + std::to_string(std::max(nring, 1)) + "], const lean_kv &kv)",
                      "lean_t");
-  emit_reset(d, net, g, "__device__ inline void lean_reset(lean_t (&x)[LEAN_M])");
+  emit_reset(d, k, "__device__ inline void lean_reset(lean_t (&x)[LEAN_M], const lean_kv &kv)");
   if (g.upd == UPD_PROGRAM) {
     // t = n dt (Clock._t, brian/clock.py:186)
-    d << "__device__ inline void lean_update(lean_t (&x)[LEAN_M], int64_t n) {\n"
+    d << "__device__ inline void lean_update(lean_t (&x)[LEAN_M], int64_t n, const lean_kv &) {\n"
       << "  program_step_code<LEAN_M>(x, (double)n * " << lit(net->dt, false) << " + 0.0, " << lit(net->dt, false)
       << ");\n}\n";
   } else {
-    emit_linear(d, net, g, "__device__ inline void lean_update(lean_t (&x)[LEAN_M], int64_t n)", "lean_t");
+    emit_linear(d, k, "__device__ inline void lean_update(lean_t (&x)[LEAN_M], int64_t n, const lean_kv &kv)", "lean_t");
   }
-  emit_spike(d, net, g, "__device__ inline bool lean_spike(const lean_t (&x)[LEAN_M])");
+  emit_spike(d, k, "__device__ inline bool lean_spike(const lean_t (&x)[LEAN_M], const lean_kv &kv)");
   d << "}\n#include \"" << kernel_header << "\"\n";
   return d.str();
 }
@@ -719,9 +802,13 @@ JitKernel jit_sweep(bm_net *net, const HostGroup &g, int K) {
 // Compiles a kernel source with the kernel headers (or takes it from the
 // cache) and loads the kernel `name`.
 JitKernel jit_compile(const std::string &src, const std::string &name) {
-  std::lock_guard<std::mutex> lk(g_jit_mu);
-  auto it = g_jit.find(src);
-  if (it != g_jit.end()) return it->second;
+  JitCache &cache = jit_cache();
+  std::lock_guard<std::mutex> lk(cache.mu);
+  auto it = cache.kernels.find(src);
+  if (it != cache.kernels.end()) {
+    it->second.mod->used = ++cache.clock;
+    return it->second;
+  }
   hiprtcProgram prog;
   if (hiprtcCreateProgram(&prog, src.c_str(), "sweep_jit.hip", kJitNumHeaders, kJitHeaders, kJitHeaderNames) !=
       HIPRTC_SUCCESS)
@@ -749,9 +836,13 @@ JitKernel jit_compile(const std::string &src, const std::string &name) {
   hiprtcDestroyProgram(&prog);
   BM_REQUIRE(!low.empty(), "specialised sweep kernel: no lowered name");
   JitKernel k;
-  BM_HIP(hipModuleLoadData(&k.mod, code.data()));
-  BM_HIP(hipModuleGetFunction(&k.fn, k.mod, low.c_str()));
-  g_jit[src] = k;
+  k.mod = std::make_shared<JitModule>();
+  BM_HIP(hipModuleLoadData(&k.mod->mod, code.data()));
+  BM_HIP(hipModuleGetFunction(&k.fn, k.mod->mod, low.c_str()));
+  k.mod->used = ++cache.clock;
+  ++cache.compiled;
+  cache.kernels[src] = k;
+  jit_trim(cache);
   return k;
 }
 
@@ -1146,12 +1237,14 @@ std::string small_source(bm_net *net) {
     for (size_t r = 0; r < 4; ++r)
       d << (r ? "," : "") << (r < g.ring_desc.size() && g.ring_desc[r].kind == RING_COUNT ? "true" : "false");
     d << "};\n";
-    emit_deliver_rings(d, net, g, "  static __device__ inline void deliver" + arr +
-                       ", const uint32_t (&w)[MAXRING], const T (&f)[MAXRING])", "T");
+    const Consts k = consts(net, g);
+    emit_values(d, k, "KV", "T");
+    emit_deliver_rings(d, k, "  static __device__ inline void deliver" + arr +
+                       ", const uint32_t (&w)[MAXRING], const T (&f)[MAXRING], const KV &kv)", "T");
     if (M > 0) {
-      emit_reset(d, net, g, "  static __device__ inline void reset" + arr + ")");
-      emit_linear(d, net, g, "  static __device__ inline void update" + arr + ")", "T");
-      emit_spike(d, net, g, "  static __device__ inline bool spike(const T (&x)[" + std::to_string(M) + "])");
+      emit_reset(d, k, "  static __device__ inline void reset" + arr + ", const KV &kv)");
+      emit_linear(d, k, "  static __device__ inline void update" + arr + ", const KV &kv)", "T");
+      emit_spike(d, k, "  static __device__ inline bool spike(const T (&x)[" + std::to_string(M) + "], const KV &kv)");
     }
     d << "};\n";
   }
@@ -1181,7 +1274,7 @@ std::string small_source(bm_net *net) {
     << "  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;\n"
     << "  if (tid < 2 * SMALL_GROUPS) cnt[tid] = 0;\n";
   for (int gi = 0; gi < ng; ++gi)
-    d << "  SmallRegs<SG" << gi << "> r" << gi << ";\n  SmallRaster rr" << gi << " = {0};\n  const int D" << gi
+    d << "  const SG" << gi << "::KV kv" << gi << "(gd[" << gi << "]);\n  SmallRegs<SG" << gi << "> r" << gi << ";\n  SmallRaster rr" << gi << " = {0};\n  const int D" << gi
       << " = gd[" << gi << "].D, N" << gi << " = (int)gd[" << gi << "].N;\n  int sl" << gi << " = (int)(n0 % D" << gi
       << ");\n  small_load<SG" << gi << ">(gd[" << gi << "], r" << gi << ", sm, sn, tid);\n";
   for (size_t s = 0; s < net->stdps.size(); ++s)
@@ -1193,7 +1286,7 @@ std::string small_source(bm_net *net) {
     return "(sl" + i + " == 0 ? D" + i + " - 1 : sl" + i + " - 1)";
   };
   for (int gi = 0; gi < ng; ++gi)
-    d << "    small_sweep<SG" << gi << ">(gd[" << gi << "], r" << gi << ", sm, sn, n, tail, " << before(gi) << ", c + " << gi
+    d << "    small_sweep<SG" << gi << ">(gd[" << gi << "], kv" << gi << ", r" << gi << ", sm, sn, n, tail, " << before(gi) << ", c + " << gi
       << ", tid);\n";
   for (size_t s = 0; s < net->stdps.size(); ++s)
     d << "    small_decay<" << T << ">(sd[" << s << "], sm, sn, " << s << ", tid);\n";
@@ -1218,7 +1311,7 @@ std::string small_source(bm_net *net) {
   for (int gi = 0; gi < ng; ++gi) d << "    if (++sl" << gi << " == D" << gi << ") sl" << gi << " = 0;\n";
   d << "  }\n";
   for (int gi = 0; gi < ng; ++gi)
-    d << "  small_finish<SG" << gi << ">(gd[" << gi << "], r" << gi << ", sm, sn, n0 + nsteps, " << before(gi) << ", tid);\n";
+    d << "  small_finish<SG" << gi << ">(gd[" << gi << "], kv" << gi << ", r" << gi << ", sm, sn, n0 + nsteps, " << before(gi) << ", tid);\n";
   d << "  __syncthreads();\n";
   for (int gi = 0; gi < ng; ++gi) {
     d << "  small_store<SG" << gi << ">(gd[" << gi << "], r" << gi << ", sm, sn, tid);\n";
@@ -3000,6 +3093,11 @@ int bm_net_get_tuning(bm_net *net, int key, int *value) {
       case BM_TUNE_PERSIST_QUEUE: *value = net->persist_queue; break;
       case BM_TUNE_ROUTE: *value = net->route; break;
       case BM_TUNE_SMALL: *value = net->small_req; break;
+      case BM_TUNE_COMPILED: {
+        std::lock_guard<std::mutex> lk(jit_cache().mu);
+        *value = (int)jit_cache().compiled;
+        break;
+      }
       default: throw Error(BM_EINVAL, "unknown tuning key");
     }
   });

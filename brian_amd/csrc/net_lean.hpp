@@ -8,18 +8,19 @@
 //   lean_t                     the arithmetic type (float or double)
 //   LEAN_M                     state variables
 //   LEAN_NRING, lean_count[], lean_sw[]   the rings: counts (else floats), bytes per neuron
-//   lean_deliver_rings(x, w, f)  applies a step's slices of all rings (w count words, f floats)
+//   lean_kv                    the constants that come from the descriptor (none in
+//                              the common shape, whose constants are literals)
+//   lean_deliver_rings(x, w, f, kv)  applies a step's slices of all rings (w count words, f floats)
 //   LEAN_POISSON               1: Poisson sources instead of neurons (no state, no rings)
-//   lean_reset(x)              the reset ops (brian/reset.py:139-147)
-//   lean_update(x, n)          step n: S <- A.S + C with A and C as literals, or
+//   lean_reset(x, kv)          the reset ops (brian/reset.py:139-147)
+//   lean_update(x, n, kv)      step n: S <- A.S + C, or
 //                              the integration scheme's step of the program
 //   LEAN_WMAX                  the widest window the network's delays allow: what
 //                              the step loop is unrolled to (a network without
 //                              delays, one step: 7.1 -> 6.4 us a step at 4000
 //                              neurons in FP64 against 16 guarded copies)
-//   LEAN_EMP                   EmpiricalThreshold's period in steps
-//                              (brian/threshold.py:409-457), -1: none
-//   lean_spike(x)              the threshold condition (brian/threshold.py:160-191)
+//   LEAN_EMP                   1: EmpiricalThreshold (brian/threshold.py:409-457)
+//   lean_spike(x, kv)          the threshold condition (brian/threshold.py:160-191)
 //   LEAN_REFR                  1: Refractoriness (brian/reset.py:311-332), the
 //                              reset op held while step - last spike < period
 //                              and the threshold gated by last + refractory <= t;
@@ -43,7 +44,7 @@
 #define LEAN_REFR 0
 #endif
 // the last spike step of each neuron is followed within the window
-#define LEAN_LAST (LEAN_REFR || LEAN_EMP >= 0)
+#define LEAN_LAST (LEAN_REFR || LEAN_EMP)
 
 namespace bm {
 
@@ -64,6 +65,9 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
   const int N = (int)g.N;
   const int blk0 = blockIdx.x * (BLOCK * K);
   const int nsteps = tail_only ? 1 : W;
+#if !LEAN_POISSON
+  const lean_kv kv(g);
+#endif
 
   T s[K][MM];
   int32_t last[K], last0[K];
@@ -165,7 +169,7 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
 #pragma unroll
       for (int k = 0; k < K; ++k) {
 #if LEAN_NRING > 0
-        lean_deliver_rings(s[k], cw[w][k], fw[w][k]);
+        lean_deliver_rings(s[k], cw[w][k], fw[w][k], kv);
 #endif
 #if LEAN_REFR
         // the tail of step n0 + w - 1: the reset holds for `period` steps
@@ -173,13 +177,13 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
         if (lastw[k] != NEVER && (n0 + w - 1) - (int64_t)lastw[k] < (int64_t)g.period) {
 #if LEAN_REFR == 2
           const double na = (double)lastw[k] * g.dt + rtime[k];
-          if (na > ((double)(n0 + w - 1) * g.dt - g.dt * 0.25)) lean_reset(s[k]);
+          if (na > ((double)(n0 + w - 1) * g.dt - g.dt * 0.25)) lean_reset(s[k], kv);
 #else
-          lean_reset(s[k]);
+          lean_reset(s[k], kv);
 #endif
         }
 #else
-        if (prev[k]) lean_reset(s[k]);
+        if (prev[k]) lean_reset(s[k], kv);
 #endif
       }
     }
@@ -195,11 +199,11 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
         t = g.ptab[g.ptab_per_neuron ? row * N + (blk0 + k * BLOCK + tid) : row];
       bool sp = valid[k] && (uint64_t)(uint32_t)(counter_u64(key[k], (uint64_t)(n0 + w)) >> 32) < t;
 #else
-      lean_update(s[k], n0 + w);
-      bool sp = valid[k] && lean_spike(s[k]);
+      lean_update(s[k], n0 + w, kv);
+      bool sp = valid[k] && lean_spike(s[k], kv);
 #endif
-#if LEAN_EMP >= 0
-      if (lastw[k] != NEVER && (n0 + w) - (int64_t)lastw[k] <= LEAN_EMP) sp = false;
+#if LEAN_EMP
+      if (lastw[k] != NEVER && (n0 + w) - (int64_t)lastw[k] <= (int64_t)g.th_period) sp = false;
 #endif
 #if LEAN_REFR
       if (sp && lastw[k] != NEVER) {

@@ -261,6 +261,7 @@ __device__ __attribute__((always_inline)) inline void persist_network(const Grou
   constexpr int NW = PBLOCK / 64;  // wavefronts
   using T = lean_t;
   constexpr int M = LEAN_M;
+  const lean_kv kv(g);
   constexpr int KR = K - KL;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -343,7 +344,7 @@ __device__ __attribute__((always_inline)) inline void persist_network(const Grou
     }                                                                                            \
     T r[M];                                                                                      \
     _Pragma("unroll") for (int j = 0; j < M; ++j) r[j] = x[j];                                   \
-    lean_reset(r);                                                                               \
+    lean_reset(r, kv);                                                                           \
     const bool rs = (prev >> (k)) & 1u;                                                          \
     _Pragma("unroll") for (int j = 0; j < M; ++j) x[j] = rs ? r[j] : x[j];                       \
   }
@@ -378,9 +379,9 @@ __device__ __attribute__((always_inline)) inline void persist_network(const Grou
     uint32_t nzk = 0u;  // its slots with spikes
 #define PERSIST_HEAD(k, x)                                                                       \
   {                                                                                              \
-    lean_update(x, n);                                                                           \
+    lean_update(x, n, kv);                                                                       \
     PERSIST_PUT(k, x)                                                                            \
-    const bool sp = ((valid >> (k)) & 1u) && lean_spike(x);                                      \
+    const bool sp = ((valid >> (k)) & 1u) && lean_spike(x, kv);                                  \
     const unsigned long long mask = __ballot(sp);                                                \
     prev = (prev & ~(1u << (k))) | ((uint32_t)sp << (k));                                        \
     if (mask != 0ull) {                                                                          \

@@ -111,7 +111,7 @@ __device__ inline void small_store(const GroupDev &g, SmallRegs<G> &r, unsigned 
 
 // Tail of step n-1 for neuron i, slot k: deliveries of ring slot sl, resets.
 template <class G>
-__device__ inline void small_tail(const GroupDev &g, SmallRegs<G> &r, unsigned char *sm, const SmallNet &sn, int64_t n,
+__device__ inline void small_tail(const GroupDev &g, const typename G::KV &kv, SmallRegs<G> &r, unsigned char *sm, const SmallNet &sn, int64_t n,
                                   int sl, int k, int i) {
   using T = typename G::T;
   uint32_t w[MAXRING];
@@ -129,23 +129,23 @@ __device__ inline void small_tail(const GroupDev &g, SmallRegs<G> &r, unsigned c
       small_floats<G>(sm, sn, q)[at] = (T)0;
     }
   }
-  G::deliver(r.x[k], w, f);
+  G::deliver(r.x[k], w, f, kv);
   if (r.last[k] == NEVER) return;
   if constexpr (G::REFR == 0) {
-    if (r.last[k] == (int32_t)(n - 1)) G::reset(r.x[k]);
+    if (r.last[k] == (int32_t)(n - 1)) G::reset(r.x[k], kv);
   } else if ((n - 1) - (int64_t)r.last[k] < (int64_t)g.period) {
     if constexpr (G::REFR == 2) {
       const double na = (double)r.last[k] * g.dt + g.refr_arr[i];
-      if (na > ((double)(n - 1) * g.dt - g.dt * 0.25)) G::reset(r.x[k]);
+      if (na > ((double)(n - 1) * g.dt - g.dt * 0.25)) G::reset(r.x[k], kv);
     } else {
-      G::reset(r.x[k]);
+      G::reset(r.x[k], kv);
     }
   }
 }
 
 // Phase 1 of a group: tail of step n-1 (unless skipped), head of step n.
 template <class G>
-__device__ inline void small_sweep(const GroupDev &g, SmallRegs<G> &r, unsigned char *sm, const SmallNet &sn, int64_t n,
+__device__ inline void small_sweep(const GroupDev &g, const typename G::KV &kv, SmallRegs<G> &r, unsigned char *sm, const SmallNet &sn, int64_t n,
                                    bool tail, int sl, int *cnt, int tid) {
   const int N = (int)g.N, lane = tid & 63;
   uint16_t *list = reinterpret_cast<uint16_t *>(sm + sn.list_off[G::GI]);
@@ -160,9 +160,9 @@ __device__ inline void small_sweep(const GroupDev &g, SmallRegs<G> &r, unsigned 
         if (g.ptab && row >= 0 && row < g.ptab_len) thr = g.ptab[g.ptab_per_neuron ? row * N + i : row];
         sp = (uint64_t)counter_u32(g.seed, (uint64_t)i, (uint64_t)n) < thr;
       } else {
-        if (tail) small_tail<G>(g, r, sm, sn, n, sl, k, i);
-        G::update(r.x[k]);
-        sp = G::spike(r.x[k]);
+        if (tail) small_tail<G>(g, kv, r, sm, sn, n, sl, k, i);
+        G::update(r.x[k], kv);
+        sp = G::spike(r.x[k], kv);
         if constexpr (G::REFR != 0) {
           if (sp && r.last[k] != NEVER) {
             // next allowed spike time in seconds, as the general sweep tests it
@@ -186,12 +186,12 @@ __device__ inline void small_sweep(const GroupDev &g, SmallRegs<G> &r, unsigned 
 
 // The last tail of a run.
 template <class G>
-__device__ inline void small_finish(const GroupDev &g, SmallRegs<G> &r, unsigned char *sm, const SmallNet &sn,
+__device__ inline void small_finish(const GroupDev &g, const typename G::KV &kv, SmallRegs<G> &r, unsigned char *sm, const SmallNet &sn,
                                     int64_t n, int sl, int tid) {
   if constexpr (!G::POISSON) {
 #pragma unroll
     for (int k = 0; k < G::K; ++k)
-      if (k * SMT + tid < (int)g.N) small_tail<G>(g, r, sm, sn, n, sl, k, k * SMT + tid);
+      if (k * SMT + tid < (int)g.N) small_tail<G>(g, kv, r, sm, sn, n, sl, k, k * SMT + tid);
   }
 }
 

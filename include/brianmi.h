@@ -370,7 +370,13 @@ int bm_net_set_partition(bm_net *net, int gid, int nparts, const int64_t *offset
  *                              yet, BM_ROUTE_WINDOWS (a launch per group and
  *                              window), BM_ROUTE_ONE_WORKGROUP (the whole network
  *                              in one), or the threads of the largest network's
- *                              workgroup in a persistent launch */
+ *                              workgroup in a persistent launch
+ *   BM_TUNE_COMPILED           (get only) kernels compiled at run time so far by
+ *                              this process, whatever the handle.  They are kept
+ *                              while a handle uses them, and the last 32 others;
+ *                              networks that differ only in the constants of
+ *                              groups with several rings, float rings, empirical
+ *                              thresholds or more than 4 variables share them */
 enum {
   BM_TUNE_WINDOW = 1,
   BM_TUNE_NEURONS_PER_THREAD = 2,
@@ -387,7 +393,8 @@ enum {
   BM_TUNE_PERSIST_CHUNK = 13,
   BM_TUNE_PERSIST_QUEUE = 14,
   BM_TUNE_ROUTE = 15,
-  BM_TUNE_SMALL = 16
+  BM_TUNE_SMALL = 16,
+  BM_TUNE_COMPILED = 17
 };
 enum { BM_ROUTE_WINDOWS = 1, BM_ROUTE_ONE_WORKGROUP = 2 };
 int bm_net_set_tuning(bm_net *net, int key, int value);
