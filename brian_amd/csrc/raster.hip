@@ -14,10 +14,12 @@
 // a 2^20-neuron network take four passes over 5 MB, about 0.12 ms in 13
 // kernels, bound by their launches and by the copy to the host after them:
 // running 2000 steps and reading raster and state takes 13.6 ms, and took
-// 57.7 with the copied regions sorted on the host (std::sort).  4096 is what
-// one workgroup sorts in about the time three launches take; the 500 spikes
-// of 200 steps of 4000 neurons: 1.29 -> 1.08 ms for the run and its reading,
-// most of it one copy in place of one per region.
+// 57.7 with the copied regions sorted on the host (std::sort).  4096 entries
+// fill 32 KiB of LDS; up to there one workgroup is the faster way: a read with
+// its copies takes 85 us so and 130 by radix passes for 100 entries, 114 and 150 to
+// 174 (two to four passes) for 4096.  The 500 spikes of 200 steps of 4000
+// neurons: 1.29 -> 1.08 ms for the run and its reading, most of it one copy in
+// place of one per region.
 #include "net_launch.hpp"
 
 #include <algorithm>

@@ -2,6 +2,7 @@
 index), repeats kept, at the sizes where the path changes (one workgroup's
 LDS, one tile of the radix sort, several tiles, 64-bit keys), against numpy's
 sort of the generator's table."""
+import ctypes as C
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -57,4 +58,30 @@ def test_rasters_read_by_several_threads():
         for g, r in reads:
             np.testing.assert_array_equal(r.result()[0], want[g][0])
             np.testing.assert_array_equal(r.result()[1], want[g][1])
+    h.close()
+
+
+def _free_bytes():
+    hip = C.CDLL("libamdhip64.so.7")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_large_raster_gives_its_buffers_back():
+    """8 million spikes need 128 MB to sort; the handle does not keep them."""
+    n, steps = 1 << 20, 8
+    h = NetHandle(1e-4, 32)
+    g = h.add_group(np.ones((1, n)))
+    h.set_linear(g, np.eye(1), np.zeros(1))
+    h.set_threshold(g, 0, 0.5)
+    h.record(g, n * steps)
+    h.prepare()
+    h.run(steps)
+    h.sync()
+    before = _free_bytes()
+    s, i = h.get_spikes(g)
+    assert abs(before - _free_bytes()) < 64 << 20
+    np.testing.assert_array_equal(s, np.repeat(np.arange(steps), n))
+    np.testing.assert_array_equal(i, np.tile(np.arange(n), steps))
     h.close()
