@@ -54,6 +54,15 @@ __host__ __device__ inline uint32_t weyl_u32(uint32_t key, uint32_t counter) {
 }
 
 #if defined(__HIPCC__) || defined(__HIPCC_RTC__)
+// The logarithm of nonlinear models.  A process's run-time compiler is the one it
+// loaded first (a process with torch takes torch's), whose device functions are not
+// always those the library was built with: of ROCm 7.0's and 7.2's exp, log, pow,
+// sin, cos, tanh and sqrt in both precisions, the FP32 logarithm alone differs, by
+// one unit in the last place for 1 % of the values.  Rounded from the FP64
+// logarithm, it has the same bits whoever compiles it, interpreted and compiled.
+__device__ __forceinline__ float prog_log(float x) { return (float)log((double)x); }
+__device__ __forceinline__ double prog_log(double x) { return log(x); }
+
 // a value that is the same in all lanes, in a scalar register
 __device__ __forceinline__ float uniform(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));

@@ -544,7 +544,7 @@ std::string prog_prelude(bm_net *net, const HostGroup &g) {
       case OP_DIV: e = a + " / " + b; break;
       case OP_NEG: e = "-" + a; break;
       case OP_EXP: e = "exp(" + a + ")"; break;
-      case OP_LOG: e = "log(" + a + ")"; break;
+      case OP_LOG: e = "prog_log(" + a + ")"; break;
       case OP_SQRT: e = "sqrt(" + a + ")"; break;
       case OP_POW: e = "pow(" + a + ", " + b + ")"; break;
       case OP_ABS: e = "fabs(" + a + ")"; break;

@@ -94,7 +94,7 @@ __device__ inline void run_program(const ProgDev &p, T *reg, int tid, double t) 
       case OP_DIV: *rd = ra / rb; break;
       case OP_NEG: *rd = -ra; break;
       case OP_EXP: *rd = exp(ra); break;
-      case OP_LOG: *rd = log(ra); break;
+      case OP_LOG: *rd = prog_log(ra); break;
       case OP_SQRT: *rd = sqrt(ra); break;
       case OP_POW: *rd = pow(ra, rb); break;
       case OP_ABS: *rd = fabs(ra); break;
