@@ -3183,6 +3183,14 @@ namespace {
 // million); larger ones are released after the read, whose copy to the host takes
 // milliseconds against the 0.1 or so of allocating them.
 constexpr size_t RASTER_KEEP = size_t(64) << 20;
+// Rasters of so few entries in so few regions are sorted on the host: a region is
+// one copy of 12 us or more, and its entries are in order but for a few.  us a
+// read, host / device: 1 region of 256 entries 67 / 83, of 3968 82 / 125, of 8000
+// 111 / 162, of 40,000 393 / 334; 2 regions 256 80 / 91, 7936 119 / 140, 16,000 327 /
+// 145; 4 regions 32 100 / 81, 3840 122 / 116.  (A small network's one workgroup
+// fills a region with 512 entries before it takes the next.)
+constexpr int RASTER_HOST_REGIONS = 2;
+constexpr int64_t RASTER_HOST = 8192;
 
 // Total of the regions' counters, none of which may have overflowed.
 int64_t checked_total(HostGroup &g, const std::vector<unsigned long long> &cs) {
@@ -3229,9 +3237,12 @@ int bm_net_get_spikes(bm_net *net, int gid, int32_t *steps, int32_t *idx, int64_
     BM_REQUIRE(c <= cap, "output buffer too small");
     *n_out = c;
     if (c == 0) return;
-    // sorted on the device, unless its buffers do not fit there
+    // sorted on the device, unless its buffers do not fit there or the few
+    // regions in use are copied and sorted sooner
     const size_t want = raster_sort_bytes(c, g.raster_first, net->step, g.N);
-    bool fits = c < (int64_t(1) << 31);
+    int filled = 0;
+    for (unsigned long long q : cs) filled += q > 0;
+    bool fits = c < (int64_t(1) << 31) && !(filled <= RASTER_HOST_REGIONS && c <= RASTER_HOST);
     std::unique_lock<std::mutex> lk(net->raster_mu);
     if (fits && net->raster_work.bytes < want) {
       try {

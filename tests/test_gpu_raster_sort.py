@@ -61,6 +61,31 @@ def test_rasters_read_by_several_threads():
     h.close()
 
 
+@pytest.mark.parametrize("regions", [1, 2, 3])
+@pytest.mark.parametrize("n", [1, 30, 4095, 4200, 8190, 8195, 12000])
+def test_few_regions(regions, n):
+    """A workgroup of 256 neurons appends to a region: up to 2 of them and 8192
+    entries are sorted on the host, others on the device."""
+    rng = np.random.default_rng(n)
+    N = 256 * regions
+    per = min(n, 30 * regions)                # neurons that spike at every step
+    who = np.sort(rng.permutation(N)[:per])
+    S0 = np.zeros((1, N))
+    S0[0, who] = 2
+    h = NetHandle(1e-4, 32)
+    g = h.add_group(S0)
+    h.set_linear(g, np.eye(1), np.zeros(1))
+    h.set_threshold(g, 0, 1.0)
+    h.record(g, 2 * n + 64)
+    h.prepare()
+    steps = max(1, n // per)
+    h.run(steps)
+    s, i = h.get_spikes(g)
+    np.testing.assert_array_equal(s, np.repeat(np.arange(steps), per))
+    np.testing.assert_array_equal(i, np.tile(who, steps))
+    h.close()
+
+
 def _free_bytes():
     hip = C.CDLL("libamdhip64.so.7")
     free, total = C.c_size_t(), C.c_size_t()
