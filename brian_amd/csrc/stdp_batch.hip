@@ -25,13 +25,16 @@
 // FP32 weights are accumulated with Kahan compensation; FP64 (check mode)
 // uses plain adds.
 //
-// Bound by the vector unit: a 1024 x 1000 FP32 step at 4 x 4 issues 70 VALU
+// Bound by the vector unit: a 1024 x 1000 FP32 step at 4 x 4 issues 65 VALU
 // instructions a wavefront, eight of them quarter-rate multiplies, which fill
-// 376 of the 491 cycles that each of a SIMD's four wavefronts has in a step of
-// 0.83 us at 2.37 GHz (counters over 20,000 steps).  93 of them took 0.96 us
+// 357 of the 434 cycles that each of a SIMD's four wavefronts has in a step of
+// 0.73 us at 2.37 GHz (counters over 20,000 steps).  93 of them took 0.96 us
 // a step; scalar lane masks for the spikes, one branch over a wavefront's four
 // slots, first list entries read ahead of the draws and variable indices known
-// at compile time make it 0.84.
+// at compile time make it 0.84, the masks as lane predicates instead of a 64-bit
+// shift per lane 0.73.  At higher rates lists hold more than an entry: a second
+// read of the first one, and the shifts, made 1000 steps of 256 x 1000 at 100 Hz
+// 1.54 ms where plain code took 1.42; without them 1.31 (at 500 Hz all three 3.14).
 #include "common.hpp"
 #include "../../include/brianmi.h"
 
@@ -203,7 +206,7 @@ __global__ __launch_bounds__(64 * NW) void k_stdp_batch(const StdpBatchDev d, in
           if (mask == 0ull) continue;
           const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-          if ((mask >> lane) & 1ull) list[cnt + below] = rw[j];
+          if (__builtin_amdgcn_inverse_ballot_w64(mask)) list[cnt + below] = rw[j];
           cnt += __popcll(mask);
         }
       } else if (lane == 0) {
@@ -235,7 +238,8 @@ __global__ __launch_bounds__(64 * NW) void k_stdp_batch(const StdpBatchDev d, in
         for (int v = 0; v < NW; ++v) {
           const int c = (int)((words[v / 2] >> (16 * (v & 1))) & 0xFFFFu);
           const T *lv = sh_list + (b * NW + v) * 64 * NJ;
-          for (int k = 0; k < c; ++k) x = x + lv[k];
+          x = x + head[v];
+          for (int k = 1; k < c; ++k) x = x + lv[k];
         }
       }
     }
@@ -246,7 +250,7 @@ __global__ __launch_bounds__(64 * NW) void k_stdp_batch(const StdpBatchDev d, in
     if (any != 0ull)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-      if (spk[j] == 0ull || !((spk[j] >> lane) & 1ull)) continue;
+      if (spk[j] == 0ull || !__builtin_amdgcn_inverse_ballot_w64(spk[j])) continue;
       ra[j] = (d.interactions == 0 || d.interactions == 3) ? ra[j] + Ap : Ap;
       if (d.update == 0 && KAHAN) {
         const T y = apost - rc[j];
