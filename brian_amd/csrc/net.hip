@@ -743,6 +743,7 @@ std::string lean_prelude(bm_net *net, const HostGroup &g, const char *kernel_hea
     << "}, lean_sw[] = {" << each([](const RingDev &r) { return r.sw; }) << "};\n#define LEAN_EMP " << (g.th_kind == TH_EMPIRICAL ? 1 : 0) << "\n#define LEAN_M " << M << "\n#define LEAN_SW " << sw
     << "\n#define LEAN_REFR " << (g.refr == REFR_CONST ? 1 : (g.refr == REFR_ARRAY ? 2 : 0)) << "\n";
   const Consts k = consts(net, g);
+  d << "#define LEAN_PERIOD " << (k.table ? std::string("(int64_t)g.th_period") : std::to_string(g.th_period)) << "\n";
   emit_values(d, k, "lean_kv", "lean_t");
   if (g.kind == GK_POISSON) {
     d << "}\n#include \"" << kernel_header << "\"\n";

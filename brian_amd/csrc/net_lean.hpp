@@ -19,7 +19,8 @@
 //                              the step loop is unrolled to (a network without
 //                              delays, one step: 7.1 -> 6.4 us a step at 4000
 //                              neurons in FP64 against 16 guarded copies)
-//   LEAN_EMP                   1: EmpiricalThreshold (brian/threshold.py:409-457)
+//   LEAN_EMP                   1: EmpiricalThreshold of LEAN_PERIOD steps
+//                              (brian/threshold.py:409-457)
 //   lean_spike(x, kv)          the threshold condition (brian/threshold.py:160-191)
 //   LEAN_REFR                  1: Refractoriness (brian/reset.py:311-332), the
 //                              reset op held while step - last spike < period
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(BLOCK) void k_lean(const GroupDev g, const int64_t 
       bool sp = valid[k] && lean_spike(s[k], kv);
 #endif
 #if LEAN_EMP
-      if (lastw[k] != NEVER && (n0 + w) - (int64_t)lastw[k] <= (int64_t)g.th_period) sp = false;
+      if (lastw[k] != NEVER && (n0 + w) - (int64_t)lastw[k] <= LEAN_PERIOD) sp = false;
 #endif
 #if LEAN_REFR
       if (sp && lastw[k] != NEVER) {
