@@ -854,6 +854,15 @@ JitKernel jit_compile(const std::string &src, const std::string &name) {
   return k;
 }
 
+// Forgets the captured launches, which hold what they were captured with.
+void drop_graph(bm_net *net) {
+  if (!net->graph_exec) return;
+  BM_HIP(hipStreamSynchronize(net->stream));
+  hipGraphExecDestroy(net->graph_exec);
+  net->graph_exec = nullptr;
+  net->graph_windows = 0;
+}
+
 // Compiles (or takes from the cache) the specialised lean kernel of every
 // group for the current neurons-per-thread; called before any launch or
 // graph capture.
@@ -865,6 +874,7 @@ void ensure_jit(bm_net *net) {
     if (kind == JIT_NONE) continue;
     const int K = group_K(net, g);
     if (g.jit_K == K && g.jit.fn && g.jit_is == kind) continue;
+    if (g.jit.fn) drop_graph(net);      // the cache may unload the kernel it launches
     g.jit = jit_sweep(net, g, K);
     g.jit_K = K;
     g.jit_is = kind;
@@ -3072,13 +3082,7 @@ int bm_net_set_tuning(bm_net *net, int key, int value) {
       default:
         throw Error(BM_EINVAL, "unknown tuning key");
     }
-    // captured launches hold the old configuration
-    if (net->graph_exec) {
-      BM_HIP(hipStreamSynchronize(net->stream));
-      hipGraphExecDestroy(net->graph_exec);
-      net->graph_exec = nullptr;
-      net->graph_windows = 0;
-    }
+    drop_graph(net);   // captured launches hold the old configuration
   });
 }
 

@@ -371,6 +371,16 @@ def test_idle_kernels_are_dropped():
     h, q = build(values[0])                   # the held network's own
     assert h.get_tuning("compiled") == compiled + 1
     np.testing.assert_array_equal(run(h, q), want)
+    # another shape: the kernel that the captured launches hold falls idle, as the
+    # one used longest ago
+    for net, gid in ((held, g), (h, q)):
+        net.set_tuning("neurons_per_thread", 2)
+        net.run(150)
+    plain, p = build(values[0])
+    plain.run(450)
+    for x, y in zip(held.get_spikes(g), plain.get_spikes(p)):
+        np.testing.assert_array_equal(x, y)
+    plain.close()
     h.close()
     held.close()
 
