@@ -332,9 +332,10 @@ int bm_net_set_partition(bm_net *net, int gid, int nparts, const int64_t *offset
  *                              1) / 2 and fixes neurons_per_thread
  *   BM_TUNE_LEAN               1 (default): a specialised group's kernel has
  *                              its model compiled in (propagator, weights,
- *                              reset and threshold values as literals; spikes
- *                              kept as per-step wavefront ballots until the end
- *                              of the window); 0: the table-driven form
+ *                              reset and threshold values as literals, outside
+ *                              the common shape read once a launch; spikes kept
+ *                              as per-step wavefront ballots until the end of
+ *                              the window); 0: the table-driven form
  *   BM_TUNE_PERSIST            (after prepare) 1: each run is one persistent
  *                              launch per group in which every network of the
  *                              group's partition (bm_net_set_partition) is
@@ -342,9 +343,9 @@ int bm_net_set_partition(bm_net *net, int gid, int nparts, const int64_t *offset
  *                              threads: the smallest that holds it where there
  *                              are more networks than compute units, else 256
  *                              for networks of at most 512 neurons and 1024 for
- *                              larger) through all the run's steps, state in registers, one
- *                              workgroup barrier per step.  Needs lean groups with count
- *                              rings, connections within a group, delays of
+ *                              larger) through all the run's steps, state in
+ *                              registers, one workgroup barrier per step.  Needs
+ *                              lean groups with count rings, connections within a group, delays of
  *                              at least one step, no STDP, networks of at
  *                              most 20,480 neurons in FP32 (16,384 for models
  *                              of more than 3 variables, 8,192 in FP64);
